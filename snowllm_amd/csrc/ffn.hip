@@ -168,16 +168,23 @@ __global__ void __launch_bounds__(NORM_MAX_THREADS) norm_prep_kernel(
 // ---------------------------------------------------------------------------------------
 constexpr int WT_F16 = 1;
 constexpr int WT_BF16 = 2;
-constexpr int DENSE_MT = 4;        // row tiles per dense_gemv workgroup above two
+constexpr int DENSE_MT = 8;        // most row tiles of a dense_gemv_wide workgroup
 constexpr int DENSE_MAX_M = 256;   // rows of one verify step
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-// One launch covers up to MT 16-row tiles of the rows (blockIdx.y: the group of MT tiles):
-// each superblock's weights are loaded once and multiplied against every tile's operands, so
-// a wide verify block streams the weights once per MT tiles. Each row's arithmetic is the
-// same whatever MT is (an MFMA row depends on its own operands only).
-template <int WT, int NTILE, int NW, int MT>
+template <int WT>
+__device__ __forceinline__ floatx4 dense_mfma(const u32x4& a, const u32x4& b, floatx4 c) {
+  if constexpr (WT == WT_F16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a),
+                                                  __builtin_bit_cast(half8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// One 16-row tile per workgroup (blockIdx.y: the row tile).
+template <int WT, int NTILE, int NW>
 __global__ void __launch_bounds__(NW * 64) dense_gemv(const u32x4* __restrict__ w,
                                                       const void* __restrict__ act,
                                                       void* __restrict__ c, int M, int N, int S,
@@ -189,39 +196,29 @@ __global__ void __launch_bounds__(NW * 64) dense_gemv(const u32x4* __restrict__ 
   const int tiles = (N + TILE_N - 1) / TILE_N;
   const int tile0 = blockIdx.x * NTILE;
   const int K = S * QK;
-  const int m0 = blockIdx.y * MT;                       // first row tile of the group
-  const int row_tiles = (M + TILE_M - 1) / TILE_M;
-  const int mt = row_tiles - m0 < MT ? row_tiles - m0 : MT;
+  const int m0 = blockIdx.y;
+  const int rows = M - m0 * TILE_M < TILE_M ? M - m0 * TILE_M : TILE_M;  // >= 1
   // the block's own tiles as the buffer: offsets stay 32-bit whatever N * K is
   const int own = tiles - tile0 < NTILE ? tiles - tile0 : NTILE;
   __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(w + (int64_t)tile0 * S * 8 * 64), 0, own * S * 8 * 64 * 16, 0x00020000);
-  __amdgpu_buffer_rsrc_t xr[MT], sr[MT];
-  uint32_t vx[MT], vs[MT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    const int rows = M - (m0 + m) * TILE_M;  // valid rows of tile m0 + m (<= 0: none)
-    if constexpr (WT == WT_F16) {
-      XPrepView xv = xprep_view((char*)act + (size_t)(m0 + m) * tile_bytes, S);
-      xr[m] = __builtin_amdgcn_make_buffer_rsrc((void*)xv.xop, 0, S * 8 * 64 * 16, 0x00020000);
-      sr[m] = __builtin_amdgcn_make_buffer_rsrc((void*)xv.scale, 0, S * 16 * 4, 0x00020000);
-      vx[m] = r < rows ? lane * 16 : 0x80000000u;
-      vs[m] = kq * 16;
-    } else {
-      const int rv = rows < TILE_M ? (rows > 0 ? rows : 0) : TILE_M;
-      xr[m] = __builtin_amdgcn_make_buffer_rsrc(
-          (void*)((const uint16_t*)act + (int64_t)(m0 + m) * TILE_M * K), 0, rv * K * 2,
-          0x00020000);
-      sr[m] = xr[m];
-      vx[m] = r < rows ? (uint32_t)(r * K * 2 + kq * 16) : 0x80000000u;
-      vs[m] = 0;
-    }
+  __amdgpu_buffer_rsrc_t xr, sr;
+  uint32_t vx, vs = 0;
+  if constexpr (WT == WT_F16) {
+    XPrepView xv = xprep_view((char*)act + (size_t)m0 * tile_bytes, S);
+    xr = __builtin_amdgcn_make_buffer_rsrc((void*)xv.xop, 0, S * 8 * 64 * 16, 0x00020000);
+    sr = __builtin_amdgcn_make_buffer_rsrc((void*)xv.scale, 0, S * 16 * 4, 0x00020000);
+    vx = r < rows ? lane * 16 : 0x80000000u;
+    vs = kq * 16;
+  } else {
+    xr = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)((const uint16_t*)act + (int64_t)m0 * TILE_M * K), 0, rows * K * 2, 0x00020000);
+    sr = xr;
+    vx = r < rows ? (uint32_t)(r * K * 2 + kq * 16) : 0x80000000u;
   }
-  floatx4 acc[MT][NTILE];
+  floatx4 acc[NTILE];
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int t = 0; t < NTILE; ++t) acc[m][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < NTILE; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
   for (int s = wv; s < S; s += NW) {
     u32x4 wb[NTILE][8];
 #pragma unroll
@@ -229,40 +226,157 @@ __global__ void __launch_bounds__(NW * 64) dense_gemv(const u32x4* __restrict__ 
 #pragma unroll
       for (int j = 0; j < 8; ++j)
         wb[t][j] = bload4(wr, lane * 16, (uint32_t)(((t * S + s) * 8 + j) * 64 * 16));
+    u32x4 xa[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if constexpr (WT == WT_F16) xa[j] = bload4(xr, vx, (uint32_t)((s * 8 + j) * 64 * 16));
+      else xa[j] = bload4(xr, vx, (uint32_t)((s * QK + j * 32) * 2));
+    }
+    floatx4 scale = {1.f, 1.f, 1.f, 1.f};
+    if constexpr (WT == WT_F16)
+      scale = __builtin_bit_cast(floatx4, bload4(sr, vs, (uint32_t)(s * 16 * 4)));
+    __builtin_amdgcn_sched_barrier(0);  // every load of the superblock before its first product
+#pragma unroll
+    for (int t = 0; t < NTILE; ++t) {
+      floatx4 sb = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sb = dense_mfma<WT>(xa[j], wb[t][j], sb);
+      acc[t] += sb * scale;
+    }
+  }
+  combine_waves<NTILE, NW>(part, acc, wv, lane);
+  for (int idx = threadIdx.x; idx < NTILE * 64; idx += NW * 64) {
+    const int t = idx >> 6, l = idx & 63;
+    const int tile = tile0 + t;
+    if (tile >= tiles) continue;
+    floatx4 v = part[0][t][l];
+#pragma unroll
+    for (int ww = 1; ww < NW; ++ww) v += part[ww][t][l];
+    const int n = tile * TILE_N + (l & 15);
+    if (n >= N) continue;
+    const int rb = m0 * TILE_M + 4 * (l >> 4);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = rb + i;
+      if (row >= M) break;
+      if (c_bf16) ((uint16_t*)c)[(int64_t)row * N + n] = f32_to_bf16(v[i]);
+      else ((float*)c)[(int64_t)row * N + n] = v[i];
+    }
+  }
+}
+
+// The same GEMV over MT 16-row tiles at once: NT column tiles per workgroup, the waves split the
+// superblocks as the one-tile form's do, and each wave multiplies the weights it loads with
+// every row tile's operands, so the weights are read once per MT row tiles, no operand is loaded
+// by two waves of a workgroup, and every row gets the one-tile form's bits (the same products
+// per superblock, the same sums over a wave's superblocks and over the waves). Both operands
+// stream one 32-wide k-step at a time, the activations DX and the weights DW steps ahead (rings
+// in registers); the rows' scales wait in LDS for the end of their superblock. Loads past a
+// wave's last superblock go out at out-of-range offsets and touch no memory. Bound: HBM, the
+// weights' bytes (nt loads, so that they do not displace the activations from L2), up to
+// about 128 rows; matrix instructions past that.
+// MI355X, 151,936 x 4096 fp16, us (four row tiles per workgroup, weights loaded a superblock at
+// a time, before): 36 rows 331 -> 300, 108 rows 710 -> 449, 256 rows 1503 -> 978; x 2048 bf16,
+// 108 rows 533 -> 378.
+// Two row groups (more than 8 row tiles) take the same columns 8 apart in dispatch order, so that
+// both land on one XCD and the second's weights come from its L2.
+template <int WT, int NT, int NW, int MT>
+__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+dense_gemv_wide(const u32x4* __restrict__ w, const void* __restrict__ act, void* __restrict__ c,
+                int M, int N, int S, int c_bf16, size_t tile_bytes, int groups) {
+  constexpr int DX = 2, DW = MT == 8 && WT == WT_F16 ? 2 : 4;  // (four would spill there)
+  __shared__ floatx4 part[NW][NT][64];
+  __shared__ __attribute__((aligned(16))) float s_scale[NW][DENSE_MT * TILE_M];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kq = lane >> 4, r = lane & 15;
+  const int tiles = (N + TILE_N - 1) / TILE_N;
+  int cb = blockIdx.x, m0 = 0;
+  if (groups == 2) {
+    m0 = (cb & 8) ? MT : 0;
+    cb = ((cb >> 4) << 3) | (cb & 7);
+  }
+  const int tile0 = cb * NT;
+  if (tile0 >= tiles) return;
+  const int K = S * QK;
+  const int own = tiles - tile0 < NT ? tiles - tile0 : NT;
+  const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(w + (int64_t)tile0 * S * 8 * 64), 0, own * S * 8 * 64 * 16, 0x00020000);
+  // activations of the group's row tiles: fp16 operands tile_bytes apart, or bf16 rows
+  const uint32_t xstep = WT == WT_F16 ? (uint32_t)tile_bytes : (uint32_t)(TILE_M * K * 2);
+  const char* xbase = (const char*)act + (size_t)m0 * xstep;
+  const __amdgpu_buffer_rsrc_t xr =
+      __builtin_amdgcn_make_buffer_rsrc((void*)xbase, 0, (int)(MT * xstep), 0x00020000);
+  uint32_t vx[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int rows = M - (m0 + m) * TILE_M;  // valid rows of tile m0 + m (<= 0: none)
+    const uint32_t at = WT == WT_F16 ? (uint32_t)(lane * 16) : (uint32_t)(r * K * 2 + kq * 16);
+    vx[m] = r < rows ? at + m * xstep : 0x80000000u;
+  }
+  const uint32_t vw = lane * 16;
+  floatx4 acc[MT][NT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[m][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  u32x4 xa[DX][MT], wb[DW][NT];
+  auto load_x = [&](int b, int s, int j) {
+    const uint32_t off = WT == WT_F16 ? (uint32_t)((s * 8 + j) * 64 * 16) : (uint32_t)((s * QK + j * 32) * 2);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) xa[b][m] = bload4(xr, s < S ? vx[m] : 0x80000000u, s < S ? off : 0u);
+  };
+  auto load_w = [&](int b, int s, int j) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      wb[b][t] = __builtin_bit_cast(
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, s < S ? vw : 0x80000000u,
+                                                       s < S ? (uint32_t)(((t * S + s) * 8 + j) * 64 * 16) : 0u,
+                                                       2 /* nt */));
+  };
+#pragma unroll
+  for (int j = 0; j < DW; ++j) load_w(j, wv, j);
+#pragma unroll
+  for (int j = 0; j < DX; ++j) load_x(j, wv, j);
+  const size_t scale_at = (size_t)((char*)xprep_view(nullptr, S).scale - (char*)nullptr);
+  for (int s = wv; s < S; s += NW) {
+    float2 sc2 = {0.f, 0.f};
+    if constexpr (WT == WT_F16)  // lane l: rows 2 (l % 8), + 1 of row tile l / 8
+      if ((lane >> 3) < MT && (m0 + (lane >> 3)) * TILE_M < M)
+        sc2 = *(const float2*)(xbase + (lane >> 3) * (size_t)xstep + scale_at + s * 64 + (lane & 7) * 8);
+    floatx4 sb[MT][NT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) sb[m][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          sb[m][t] = dense_mfma<WT>(xa[j % DX][m], wb[j % DW][t], sb[m][t]);
+      load_x(j % DX, j + DX < 8 ? s : s + NW, (j + DX) & 7);
+      load_w(j % DW, j + DW < 8 ? s : s + NW, (j + DW) & 7);
+    }
+    if constexpr (WT == WT_F16) {
+      *(float2*)&s_scale[wv][lane * 2] = sc2;  // read back by this wave only
+      __builtin_amdgcn_wave_barrier();
+    }
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-      if (m >= mt) break;  // uniform
-      u32x4 xa[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        if constexpr (WT == WT_F16) xa[j] = bload4(xr[m], vx[m], (uint32_t)((s * 8 + j) * 64 * 16));
-        else xa[j] = bload4(xr[m], vx[m], (uint32_t)((s * QK + j * 32) * 2));
-      }
       floatx4 scale = {1.f, 1.f, 1.f, 1.f};
-      if constexpr (WT == WT_F16)
-        scale = __builtin_bit_cast(floatx4, bload4(sr[m], vs[m], (uint32_t)(s * 16 * 4)));
+      if constexpr (WT == WT_F16) scale = *(const floatx4*)&s_scale[wv][m * TILE_M + 4 * kq];
 #pragma unroll
-      for (int t = 0; t < NTILE; ++t) {
-        floatx4 sb = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          if constexpr (WT == WT_F16)
-            sb = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, xa[j]),
-                                                        __builtin_bit_cast(half8, wb[t][j]), sb, 0, 0, 0);
-          else
-            sb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xa[j]),
-                                                         __builtin_bit_cast(bf16x8, wb[t][j]), sb, 0, 0, 0);
-        }
-        acc[m][t] += sb * scale;
-      }
+      for (int t = 0; t < NT; ++t) acc[m][t] += sb[m][t] * scale;
     }
+    if constexpr (WT == WT_F16) __builtin_amdgcn_wave_barrier();
   }
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
-    if (m >= mt) break;  // uniform
     if (m) __syncthreads();  // the previous tile's partials are read
-    combine_waves<NTILE, NW>(part, acc[m], wv, lane);
-    for (int idx = threadIdx.x; idx < NTILE * 64; idx += NW * 64) {
+    combine_waves<NT, NW>(part, acc[m], wv, lane);
+    for (int idx = threadIdx.x; idx < NT * 64; idx += NW * 64) {
       const int t = idx >> 6, l = idx & 63;
       const int tile = tile0 + t;
       if (tile >= tiles) continue;
@@ -1397,19 +1511,32 @@ int launch_dense(const void* w, const void* act, void* c, int M, int N, int S, i
   const int tiles = (N + TILE_N - 1) / TILE_N;
   const int row_tiles = (M + TILE_M - 1) / TILE_M;
   const size_t tb = xprep_tile_bytes(S);
-  const int groups = (tiles + NTILE - 1) / NTILE;
-  if (row_tiles == 1 || groups < 64)
+  const int blocks = (tiles + NTILE - 1) / NTILE;
+  if (row_tiles == 1 || blocks < 64) {
     // one row tile per workgroup: a narrow output (the router's 17 tiles) then still has
     // workgroups for several CUs (the same sums per row tile)
-    hipLaunchKernelGGL((dense_gemv<WT, NTILE, NW, 1>), dim3(groups, row_tiles), dim3(NW * 64), 0,
-                       s, (const u32x4*)w, act, c, M, N, S, c_bf16, tb);
-  else if (row_tiles == 2)
-    hipLaunchKernelGGL((dense_gemv<WT, NTILE, NW, 2>), dim3((tiles + NTILE - 1) / NTILE),
-                       dim3(NW * 64), 0, s, (const u32x4*)w, act, c, M, N, S, c_bf16, tb);
-  else
-    hipLaunchKernelGGL((dense_gemv<WT, NTILE, NW, DENSE_MT>),
-                       dim3((tiles + NTILE - 1) / NTILE, (row_tiles + DENSE_MT - 1) / DENSE_MT),
-                       dim3(NW * 64), 0, s, (const u32x4*)w, act, c, M, N, S, c_bf16, tb);
+    hipLaunchKernelGGL((dense_gemv<WT, NTILE, NW>), dim3(blocks, row_tiles), dim3(NW * 64), 0, s,
+                       (const u32x4*)w, act, c, M, N, S, c_bf16, tb);
+    SV_CHECK_LAUNCH();
+    return SV_OK;
+  }
+  // every row tile in one workgroup up to DENSE_MT of them, two even groups above
+  const int groups = row_tiles > DENSE_MT ? 2 : 1;
+  const int wide = (tiles + 1) / 2;
+  const dim3 grid((unsigned)(groups == 2 ? 16 * ((wide + 7) / 8) : wide));
+  auto go = [&](auto mt) {
+    hipLaunchKernelGGL((dense_gemv_wide<WT, 2, NW, decltype(mt)::value>), grid, dim3(NW * 64), 0, s,
+                       (const u32x4*)w, act, c, M, N, S, c_bf16, tb, groups);
+  };
+  switch ((row_tiles + groups - 1) / groups) {
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 3: go(std::integral_constant<int, 3>{}); break;
+    case 4: go(std::integral_constant<int, 4>{}); break;
+    case 5: go(std::integral_constant<int, 5>{}); break;
+    case 6: go(std::integral_constant<int, 6>{}); break;
+    case 7: go(std::integral_constant<int, 7>{}); break;
+    default: go(std::integral_constant<int, 8>{}); break;
+  }
   SV_CHECK_LAUNCH();
   return SV_OK;
 }
