@@ -1,0 +1,95 @@
+"""Candidate lists and rejection at the edges of their kernels' rules, bit-exact against the
+oracle: lists within one workgroup (up to 1024) and wider ones, ties, masked rows, rows that the
+LDS buffers do not hold, odd vocabularies (unaligned rows), and the search of draft tokens."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import accept as A
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows(V, seed):
+    """Logit rows: plain, narrow (crowded probabilities), few distinct values (ties), masked by
+    -inf, masked by the lowest value, all equal, one NaN and an infinity."""
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(7, V, generator=g) * 2
+    x[1] *= 0.05
+    x[2] = (x[2] * 2).round() / 2
+    keep = torch.randperm(V, generator=g)[:max(1, V // 50)]
+    for r, low in ((3, float("-inf")), (4, torch.finfo(torch.float32).min)):
+        m = torch.full((V,), low)
+        m[keep] = x[r, keep]
+        x[r] = m
+    x[5] = 1.25
+    x[6, V // 3] = float("nan")
+    x[6, V // 2] = float("-inf")
+    return x
+
+
+def _check(V, top_k, top_p, seed):
+    from snowllm_amd import ops
+    x = _rows(V, seed)
+    n = x.shape[0]
+    width = max(min(k, V) if k > 0 else V for k in top_k)
+    k = torch.tensor(top_k, dtype=torch.int32)
+    p = torch.tensor(top_p)
+    temp = torch.linspace(0.5, 1.5, n)
+    out = torch.empty(n, width, device="cuda")
+    ids = torch.empty(n, width, dtype=torch.int64, device="cuda")
+    ws = torch.empty(ops.sample_workspace_bytes(n, V, width), dtype=torch.uint8, device="cuda")
+    print(f"lists V={V} top_k={top_k} width={width}", flush=True)
+    for _ in range(2):   # a second call on the used workspace
+        ops.probabilities(x.cuda(), k.cuda(), p.cuda(), temp.cuda(), width, out, ids, ws)
+    want_p, want_ids = A.probabilities(x.numpy(), k.numpy(), p.numpy(), temp.numpy(), width)
+    assert np.array_equal(ids.cpu().numpy(), want_ids)
+    assert np.array_equal(out.cpu().numpy().view(np.uint32), want_p.view(np.uint32))
+
+
+@pytest.mark.parametrize("V", [3, 1024, 1030, 4099, 8195, 50257, 151936])
+@pytest.mark.parametrize("k", [1, 20, 257, 1024])
+def test_short_lists(gpu, V, k):
+    _check(V, [min(k, V)] * 7, [0.9, 1.0, 0.95, 0.8, 0.7, 0.5, 0.99], V + k)
+
+
+@pytest.mark.parametrize("V", [1100, 8193, 32000, 151937])
+def test_wide_lists(gpu, V):
+    """The whole vocabulary with top-p, widths between, short lists beside them."""
+    _check(V, [0, V, 0, 1025, 0, 0, 0], [0.9, 0.5, 0.95, 1.0, 0.8, 0.3, 0.999], V)
+    _check(V, [1026, 20, V - 1, 0, 0, 1050, 7], [0.9, 0.5, 1.0, 0.9, 1.0, 0.95, 1.0], V + 1)
+
+
+@pytest.mark.parametrize("p_width,q_width", [(1, 16), (20, 16), (4096, 16), (4097, 70), (9000, 9000)])
+def test_reject_searches(gpu, p_width, q_width):
+    """Draft tokens in unordered lists, present, absent and repeated (their sum), with stale
+    proposals, at the widths where the search changes form."""
+    from snowllm_amd import ops
+    g = torch.Generator().manual_seed(p_width + q_width)
+    b, k, V = 5, 4, 20000
+    p = torch.rand(b * (k + 1), p_width, generator=g)
+    p /= p.sum(-1, keepdim=True)
+    ids = torch.stack([torch.randperm(V, generator=g)[:p_width] for _ in range(b * (k + 1))])
+    cand = torch.stack([torch.randperm(V, generator=g)[:q_width] for _ in range(b * k)])
+    q = torch.rand(b * k, q_width, generator=g)
+    q /= q.sum(-1, keepdim=True)
+    rows = [r * (k + 1) + j for r in range(b) for j in range(k)]
+    drafts = ids[rows][:, p_width // 2].clone()         # in the target's list
+    cand[:, q_width // 3] = drafts                      # and in the proposal's
+    drafts[1], drafts[6] = V + 5, -1                    # nowhere
+    if p_width > 8:
+        ids[0, 3] = ids[0, p_width - 2] = drafts[0]     # repeated ids add up
+    ids[2 * (k + 1)] = torch.arange(p_width)            # a list in vocabulary order
+    drafts[2 * k] = p_width - 1
+    args = [p, ids, drafts.view(b, k), cand.view(b, k, q_width), q.view(b, k, q_width),
+            torch.tensor([4, 3, 2, 1, 0], dtype=torch.int32),
+            torch.tensor([1, 1, 1, 0, 1], dtype=torch.int32)]
+    out = torch.empty(b, k + 1, dtype=torch.int64, device="cuda")
+    acc = torch.empty(b, dtype=torch.int64, device="cuda")
+    for u in (torch.rand(b, k + 1, generator=g), torch.rand(b, k + 1, generator=g) * 0.02,
+              torch.zeros(b, k + 1)):
+        print(f"reject p_width={p_width} q_width={q_width}", flush=True)
+        ops.dflash.reject(*[x.cuda() for x in args], u.cuda(), out, acc)
+        want, wacc = A.reject(*[x.numpy() for x in args], u.numpy())
+        assert np.array_equal(acc.cpu().numpy(), wacc)
+        assert np.array_equal(out.cpu().numpy(), want)
