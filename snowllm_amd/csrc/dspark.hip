@@ -9,18 +9,29 @@
 // (the reference's PyTorch restatement: tests/test_lfm2_dspark_reference.py:143-152).
 //
 // Each row streams all of W2 ([V, rank] bf16, 78 MB at V = 151936, rank 256) once for every
-// request of the batch together: the walk is HBM-bound, one launch per block row. W2 is packed
-// so that one wave load of 1 KB gives each of 64 lanes a 16-byte chunk of its own vocabulary
-// row; each lane sums its row's products in fp64 -- exact for products of two bf16 values --
-// and rounds the sum once, so the bias does not depend on the summation order. Every
-// workgroup reduces its rows to one (value, index) key per request; the last workgroup of a
-// two-level arrival reduces the keys, writes the pick and the confidence, and the next row's
-// launch reads the pick as its latent index.
+// request of the batch together, one launch per block row. The bias that counts is the sum of
+// the bf16 products taken in fp64 -- exact -- and rounded once, but only the largest score is
+// wanted: 16 rows x 16 requests at a time the matrix cores give every bias in fp32 with a bound
+// on its error (from the sum of the products' magnitudes, a second product), hence bounds on
+// every score, and only rows whose upper bound reaches the largest lower bound seen (a few per
+// workgroup, usually one per request in all) are summed in fp64. W2 is packed in tiles of 64
+// rows, 8 values of a row per 16 bytes, so that a 16-row operand of 32 values is four runs of
+// 256 bytes. Every workgroup reduces its rows to one (value, index) key per request; the last
+// workgroup of a two-level arrival reduces the keys and writes the pick, which the next row's
+// launch reads as its latent index; one more workgroup computes the confidences.
+// Bound: the read of W2, from the 256 MB cache after the first row, and below about 50 MB the
+// chain of the row (the latent's read, the bounds, the exact sum of the workgroup's best row, the
+// two arrivals). Sharing the lower bound between workgroups was slower for up to eight requests
+// (its round trip costs what it saves). MI355X, us per block row with confidences, every sum in
+// fp64 before -> now: V = 151,936, rank 256: 29 -> 21 for one request, 45 -> 25 for four, 108 ->
+// 33 for eight, 188 -> 49 for sixteen; rank 64: 15.5 -> 15.1, 26 -> 18, 57 -> 23 for one, four,
+// eight; V = 32,000, rank 256: 19 -> 14, 33 -> 17, 61 -> 23. Masked logits (-inf, or the type's
+// lowest value) 45 -> 24 at four requests. Equal scores everywhere take the exact sums alone.
 #include "common.h"
 
 namespace {
 
-constexpr int DSP_WAVES = 4;               // waves per 64-row tile (they split the rank)
+constexpr int DSP_WAVES = 4;               // waves per workgroup, 16 rows each at a time
 constexpr int DSP_NT = DSP_WAVES * WAVE;
 constexpr int DSP_MAX_B = 16;              // requests per call
 constexpr int DSP_MAX_RANK = 512;
@@ -74,13 +85,12 @@ struct DspArgs {
   int b, rank, block, h, nwg, fp32_bias, j;
 };
 
-// Grid: G <= 1024 workgroups of 4 waves; wave k of workgroup g takes the 64-row tiles
-// 4 g + k, 4 g + k + 4 G, ... and keeps its best (value, index) key per request. Each lane sums
-// its row's products in fp64 with 8 chunk loads (128 bytes of the row) in flight.
+// Grid: G <= 1024 workgroups of 4 waves; wave k of workgroup g takes the 16-row units 4 g + k,
+// 4 g + k + 4 G, ... with the next unit's operands in flight.
 // Arrival is two-level so that no counter sees more than 32 arrivals: the workgroups of a
 // group of 32 count on the group's counter; the group's last arrival reduces the group's keys
 // and counts on the top counter, whose last arrival reduces the groups' keys and writes the
-// pick (and the confidence).
+// pick.
 constexpr int DSP_GRID = 1024, DSP_GROUP = 32, DSP_GROUPS = DSP_GRID / DSP_GROUP;
 __device__ uint64_t g_dsp_group[DSP_GROUPS];
 
@@ -101,92 +111,241 @@ __device__ __forceinline__ uint64_t dsp_load(const uint64_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// MB: a compile-time bound on the requests (1, 4 or 16), which sizes the registers.
-template <int MB>
+// The exact score of one vocabulary row for one request (L: its latent in fp32), by one wave: a
+// chunk of eight products per lane in fp64, the lanes' sums added (exact in any order), the
+// sum rounded once. The key in every lane.
+__device__ __forceinline__ uint64_t dsp_exact_key(const DspArgs& a, const float* L, int r,
+                                                  int64_t row) {
+  const int chunks = a.rank / 8, lane = threadIdx.x & (WAVE - 1);   // chunks <= 64
+  const int64_t tile = row / WAVE;
+  const int64_t rows_t = a.v - tile * WAVE < WAVE ? a.v - tile * WAVE : WAVE;
+  const uint4* src = (const uint4*)(a.w2 + tile * WAVE * (int64_t)a.rank) + row % WAVE;
+  const int c = lane < chunks ? lane : 0;
+  const uint4 q = src[c * rows_t];
+  const float x = a.base[((int64_t)r * a.block + a.j) * a.base_stride + row];
+  const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
+  double acc = 0.0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float* l = L + c * 8 + 2 * e;
+    acc += (double)(__uint_as_float(qw[e] << 16) * l[0]);        // exact bf16 x bf16
+    acc += (double)(__uint_as_float(qw[e] & 0xffff0000u) * l[1]);
+  }
+  if (lane >= chunks) acc = 0.0;
+#pragma unroll
+  for (int d = WAVE / 2; d > 0; d >>= 1)
+    acc += __builtin_bit_cast(double, shfl_xor_u64(__builtin_bit_cast(uint64_t, acc), d));
+  const float bias = a.fp32_bias ? (float)acc : bf16_from_f64(acc);
+  return argmax_key(x + bias, (uint32_t)row);
+}
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+constexpr int DSP_UNIT = 16;              // vocabulary rows of a matrix product
+constexpr int DSP_CAND = 512;             // candidates a workgroup keeps
+constexpr uint32_t DSP_BOTTOM = 0x007fffffu;  // ord_key(-inf)
+
+// KS: 32-value steps of the rank (values past the rank are zero operands).
+template <int KS>
 __global__ void __launch_bounds__(DSP_NT) dsp_markov_kernel(DspArgs a) {
   __shared__ float s_lat[4096];                  // latents f32 [b][rank], b rank <= 4096
-  __shared__ uint64_t s_key[DSP_WAVES][DSP_MAX_B];
-  __shared__ uint32_t s_flag;
-  const int t = threadIdx.x, lane = t & (WAVE - 1), w = t / WAVE;
+  __shared__ uint64_t s_best[DSP_MAX_B];
+  __shared__ uint32_t s_low[DSP_MAX_B];          // this workgroup's largest lower bound
+  __shared__ uint32_t s_up[DSP_CAND];            // candidates: upper bound (key), row, request
+  __shared__ uint32_t s_row[DSP_CAND];
+  __shared__ uint8_t s_req[DSP_CAND];
+  __shared__ uint32_t s_n, s_flag;
+  const int t = threadIdx.x, lane = t & (WAVE - 1);
+  const int w = __builtin_amdgcn_readfirstlane(t / WAVE);
   const int B = a.b, R = a.rank, j = a.j, G = a.nwg;
+  const int col = lane & 15, kq = lane >> 4, chunks = R / 8;
+  const int64_t units = (a.v + DSP_UNIT - 1) / DSP_UNIT;
+  // operand chunks 4 s + kq of the unit's rows (the tile as the buffer: chunks past the rank and
+  // units past the last read zeros without touching memory) and the unit's base logits
+  auto load_unit = [&](int64_t u, uint4 (&q)[KS], float (&x)[4]) {
+    const int64_t tile = u * DSP_UNIT / WAVE;
+    const int64_t left = a.v - tile * WAVE;
+    const int rows_t = left >= WAVE ? WAVE : left > 0 ? (int)left : 0;
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(a.w2 + (rows_t ? tile * WAVE * (int64_t)R : 0)), 0, u < units ? rows_t * R * 2 : 0,
+        0x00020000);
+    const uint32_t at = (uint32_t)((kq * rows_t + (int)(u * DSP_UNIT % WAVE) + col) * 16);
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      q[s] = __builtin_bit_cast(
+          uint4, __builtin_amdgcn_raw_buffer_load_b128(wr, at, (uint32_t)(4 * s * rows_t * 16), 0));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int64_t n = u * DSP_UNIT + 4 * kq + i;
+      x[i] = a.base[((int64_t)(col < B ? col : 0) * a.block + j) * a.base_stride +
+                    (n < a.v ? n : a.v - 1)];
+    }
+  };
+  if ((int)blockIdx.x == G) {
+    // one workgroup more when confidences are wanted: they need the row's latent, not its pick
+    for (int r = w; r < B; r += DSP_WAVES) {
+      const int64_t at = (int64_t)r * a.block + j;
+      const int64_t prev = j == 0 ? a.anchor[r] : a.out[at - 1];
+      const uint16_t* lt = prev >= 0 && prev < a.v ? a.w1 + prev * R : nullptr;
+      const uint16_t* hid = a.pre_head + at * a.ps;
+      float z = 0.f;
+#pragma unroll 16
+      for (int i = lane; i < a.h; i += WAVE) z += bf16_to_f32(hid[i]) * a.conf_w[i];
+      for (int i = lane; i < R; i += WAVE) z += (lt ? bf16_to_f32(lt[i]) : 0.f) * a.conf_w[a.h + i];
+      z = wave_sum(z);
+      if (lane == 0) {
+        if (a.conf_b) z += *a.conf_b;
+        a.confidence[at] = 1.f / (1.f + expf(-z));
+      }
+    }
+    return;
+  }
+  int64_t u = (int64_t)blockIdx.x * DSP_WAVES + w;
+  uint4 q0[KS], q1[KS];
+  float x0[4], x1[4];
+  load_unit(u, q0, x0);
+  // (a workgroup's first row scores -inf at least: the result where every score is -inf)
+  if (t < DSP_MAX_B) {
+    s_low[t] = 0u;
+    s_best[t] = argmax_key(-__builtin_huge_valf(), (uint32_t)(blockIdx.x * DSP_WAVES * DSP_UNIT));
+  }
+  if (t == 0) s_n = 0u;
   for (int i = t; i < B * R; i += DSP_NT) {
     const int r = i / R, e = i % R;
     const int64_t prev = j == 0 ? a.anchor[r] : a.out[(int64_t)r * a.block + j - 1];
     s_lat[i] = (prev >= 0 && prev < a.v) ? bf16_to_f32(a.w1[prev * R + e]) : 0.f;
   }
   __syncthreads();
-
-  const int64_t tiles = (a.v + WAVE - 1) / WAVE;
-  const int chunks = R / 8;
-  uint64_t best[MB];
+  // the requests' latents as the other operand (column col: request col)
+  bf16x8 lat[KS];
+  float top = 0.f;
+  bool subnormal = false;
 #pragma unroll
-  for (int r = 0; r < MB; ++r) best[r] = 0;
-  for (int64_t tile = (int64_t)blockIdx.x * DSP_WAVES + w; tile < tiles;
-       tile += (int64_t)G * DSP_WAVES) {
-    const int64_t rows_t = a.v - tile * WAVE < WAVE ? a.v - tile * WAVE : WAVE;
-    const int64_t row = tile * WAVE + lane;
-    const bool live = lane < rows_t;
-    const uint4* src = (const uint4*)(a.w2 + tile * WAVE * (int64_t)R) + lane;
-    double acc[MB];
+  for (int s = 0; s < KS; ++s) {
+    uint32_t l[4] = {0u, 0u, 0u, 0u};
+    if (col < B && 4 * s + kq < chunks)
 #pragma unroll
-    for (int r = 0; r < MB; ++r) acc[r] = 0.0;
-    for (int cb = 0; cb < chunks; cb += 8) {
-      uint4 q[8];
+      for (int e = 0; e < 4; ++e) {
+        const float* f = s_lat + col * R + (4 * s + kq) * 8 + 2 * e;
+        l[e] = (__float_as_uint(f[0]) >> 16) | (__float_as_uint(f[1]) & 0xffff0000u);
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        q[u] = {0u, 0u, 0u, 0u};
-        if (live && cb + u < chunks) q[u] = src[(cb + u) * rows_t];
+        for (int k = 0; k < 2; ++k) {
+          const float m = __builtin_fabsf(f[k]);
+          top = m > top ? m : top;
+          subnormal |= m > 0.f && m < 1.17549435e-38f;
+        }
       }
+    lat[s] = __builtin_bit_cast(bf16x8, uint4{l[0], l[1], l[2], l[3]});
+  }
+
+  // |fp32 sum - exact sum| <= err Sabs: every addition of the matrix cores' chain rounds by at
+  // most 2^-22 of the running magnitude (twice a binary32 ulp, whatever the order and the
+  // rounding), products are exact; tiny covers products and sums below the normal range, and
+  // weights there, should the cores take them as zero (latents there: every row is a candidate)
+  const float err = (float)(R + 8) * 2.384185791015625e-07f;
+  top = fmaxf(top, __shfl_xor(top, 16, WAVE));
+  top = fmaxf(top, __shfl_xor(top, 32, WAVE));
+  const uint64_t sub = __ballot(subnormal);
+  const float tiny = (sub >> col & 0x0001000100010001ull)
+                         ? __builtin_huge_valf() : 1e-30f + (float)R * 1.17549435e-38f * top;
+  // rounding of the bias (bf16: 2^-9 to nearest, stated as 2^-8) and of the score in fp32
+  const float rnd = a.fp32_bias ? 2.384185791015625e-07f : 3.90625e-03f, ulp = 2.384185791015625e-07f;
+  uint32_t low = 0u;  // this lane's request: the largest lower bound of the wave's rows
+  uint64_t known = 0ull;  // and its best row whose score is known
+  for (; u < units; u += (int64_t)G * DSP_WAVES) {
+    load_unit(u + (int64_t)G * DSP_WAVES, q1, x1);
+    floatx4 c = {0.f, 0.f, 0.f, 0.f}, ca = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        if (cb + u < chunks) {
-          const uint32_t qw[4] = {q[u].x, q[u].y, q[u].z, q[u].w};
-          float wv[8];
+    for (int s = 0; s < KS; ++s) {
+      const uint4 qa = {q0[s].x & 0x7fff7fffu, q0[s].y & 0x7fff7fffu, q0[s].z & 0x7fff7fffu,
+                        q0[s].w & 0x7fff7fffu};
+      const uint4 lw = __builtin_bit_cast(uint4, lat[s]);
+      const uint4 la = {lw.x & 0x7fff7fffu, lw.y & 0x7fff7fffu, lw.z & 0x7fff7fffu, lw.w & 0x7fff7fffu};
+      c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, q0[s]), lat[s], c, 0, 0, 0);
+      ca = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, qa),
+                                                   __builtin_bit_cast(bf16x8, la), ca, 0, 0, 0);
+    }
+    uint32_t up[4];
+    uint32_t best = 0u;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            wv[2 * e] = __uint_as_float(qw[e] << 16);
-            wv[2 * e + 1] = __uint_as_float(qw[e] & 0xffff0000u);
-          }
+    for (int i = 0; i < 4; ++i) {
+      const int64_t n = u * DSP_UNIT + 4 * kq + i;
+      const float x = x0[i], d = err * ca[i] + tiny;
+      const float slack = d + rnd * (__builtin_fabsf(c[i]) + d) +
+                          ulp * (__builtin_fabsf(x) + __builtin_fabsf(c[i]));
+      uint32_t lo, hi;
+      if (!(ca[i] < 1e37f)) {
+        lo = DSP_BOTTOM, hi = 0xffffffffu;  // an infinite or NaN operand: anything
+      } else if (!(__builtin_fabsf(x) <= 3.40282346638528859812e38f)) {
+        lo = ord_key(x);  // the bias is finite: NaN and -inf stay at the bottom, +inf at the top
+        hi = lo == DSP_BOTTOM ? lo : 0xffffffffu;
+      } else {
+        lo = ord_key(x + c[i] - 2.f * slack);
+        hi = ord_key(x + c[i] + 2.f * slack);
+        // a bias below a quarter ulp of the logit leaves it as it is (logits masked with a large
+        // negative value): the score is known
+        if (__builtin_fabsf(c[i]) + d < __builtin_fabsf(x) * 1.4901161193847656e-08f && col < B &&
+            n < a.v) {
+          const uint64_t key = argmax_key(x, (uint32_t)n);
+          known = key > known ? key : known;
+          lo = hi = ord_key(x);
+          if (lo > best) best = lo;
+          hi = 0u;  // no candidate
+        }
+      }
+      const bool live = col < B && n < a.v;
+      up[i] = live ? hi : 0u;
+      best = live && lo > best ? lo : best;
+    }
+    // the unit's largest lower bound of this lane's request (four lanes hold its rows)
+    uint32_t o = (uint32_t)__shfl_xor((int)best, 16, WAVE);
+    best = o > best ? o : best;
+    o = (uint32_t)__shfl_xor((int)best, 32, WAVE);
+    best = o > best ? o : best;
+    low = best > low ? best : low;
 #pragma unroll
-          for (int r = 0; r < MB; ++r) {
-            if (r < B) {
-              const float* L = s_lat + r * R + (cb + u) * 8;
-              double s0 = 0.0, s1 = 0.0;   // two chains; the sum stays exact
-#pragma unroll
-              for (int e = 0; e < 8; e += 2) {
-                s0 += (double)(wv[e] * L[e]);        // exact bf16 x bf16
-                s1 += (double)(wv[e + 1] * L[e + 1]);
-              }
-              acc[r] += s0 + s1;
-            }
-          }
+    for (int i = 0; i < 4; ++i) {
+      if (up[i] >= low && up[i] > DSP_BOTTOM) {
+        const uint32_t at = atomicAdd(&s_n, 1u);
+        if (at < DSP_CAND) {
+          s_up[at] = up[i];
+          s_row[at] = (uint32_t)(u * DSP_UNIT + 4 * kq + i);
+          s_req[at] = (uint8_t)col;
         }
       }
     }
 #pragma unroll
-    for (int r = 0; r < MB; ++r) {
-      if (r < B && live) {
-        const float bias = a.fp32_bias ? (float)acc[r] : bf16_from_f64(acc[r]);
-        const float x = a.base[((int64_t)r * a.block + j) * a.base_stride + row] + bias;
-        const uint64_t key = argmax_key(x, (uint32_t)row);
-        best[r] = key > best[r] ? key : best[r];
-      }
-    }
-  }
+    for (int s = 0; s < KS; ++s) q0[s] = q1[s];
 #pragma unroll
-  for (int r = 0; r < MB; ++r) {
-    if (r < B) {
-      const uint64_t k = wave_max_u64(best[r]);
-      if (lane == 0) s_key[w][r] = k;
+    for (int i = 0; i < 4; ++i) x0[i] = x1[i];
+  }
+  if (lane < B) atomicMax(&s_low[lane], low);
+  if (known) atomicMax((unsigned long long*)&s_best[col], (unsigned long long)known);
+  __syncthreads();
+  // the exact scores, a wave per candidate
+  if (s_n <= DSP_CAND) {  // uniform
+    for (int i = w; i < (int)s_n; i += DSP_WAVES) {
+      const int r = s_req[i];
+      if (s_up[i] < s_low[r]) continue;
+      const uint64_t key = dsp_exact_key(a, s_lat + r * R, r, s_row[i]);
+      if (lane == 0) atomicMax((unsigned long long*)&s_best[r], (unsigned long long)key);
     }
+  } else {
+    // too many near the top (equal scores): every row of this workgroup
+    for (int64_t v0 = (int64_t)blockIdx.x * DSP_WAVES; v0 < units; v0 += (int64_t)G * DSP_WAVES)
+      for (int i = w; i < DSP_WAVES * DSP_UNIT * B; i += DSP_WAVES) {
+        const int r = i / (DSP_WAVES * DSP_UNIT);
+        const int64_t row = v0 * DSP_UNIT + i % (DSP_WAVES * DSP_UNIT);
+        if (row >= a.v) continue;
+        const uint64_t key = dsp_exact_key(a, s_lat + r * R, r, row);
+        if (lane == 0) atomicMax((unsigned long long*)&s_best[r], (unsigned long long)key);
+      }
   }
   __syncthreads();
   uint64_t* wg_keys = a.partial;                          // [b][G]
   uint64_t* group_keys = a.partial + (int64_t)B * G;      // [b][groups]
   if (t < B) {
-    uint64_t m = s_key[0][t];
-    for (int i = 1; i < DSP_WAVES; ++i) m = s_key[i][t] > m ? s_key[i][t] : m;
-    __hip_atomic_store(&wg_keys[(int64_t)t * G + blockIdx.x], m, __ATOMIC_RELAXED,
+    __hip_atomic_store(&wg_keys[(int64_t)t * G + blockIdx.x], s_best[t], __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
   }
   const int group = blockIdx.x / DSP_GROUP, groups = (G + DSP_GROUP - 1) / DSP_GROUP;
@@ -201,23 +360,12 @@ __global__ void __launch_bounds__(DSP_NT) dsp_markov_kernel(DspArgs a) {
                          __HIP_MEMORY_SCOPE_AGENT);
   }
   if (!dsp_arrive(&g_dsp_cnt, groups, group == 0, &s_flag)) return;
-  // the last group: the pick and the confidence, one wave per request
+  // the last group: the pick, one wave per request
   for (int r = w; r < B; r += DSP_WAVES) {
     uint64_t m = lane < groups ? dsp_load(&group_keys[r * groups + lane]) : 0;
     m = wave_max_u64(m);
     const int64_t at = (int64_t)r * a.block + j;
     if (lane == 0) a.out[at] = (int64_t)argmax_key_index(m);
-    if (a.confidence) {
-      float z = 0.f;
-      const uint16_t* hid = a.pre_head + at * a.ps;
-      for (int i = lane; i < a.h; i += WAVE) z += bf16_to_f32(hid[i]) * a.conf_w[i];
-      for (int i = lane; i < R; i += WAVE) z += s_lat[r * R + i] * a.conf_w[a.h + i];
-      z = wave_sum(z);
-      if (lane == 0) {
-        if (a.conf_b) z += *a.conf_b;
-        a.confidence[at] = 1.f / (1.f + expf(-z));
-      }
-    }
   }
 }
 
@@ -225,6 +373,12 @@ int64_t dsp_nwg(int64_t v) {
   const int64_t tiles = (v + WAVE - 1) / WAVE;
   const int64_t g = (tiles + DSP_WAVES - 1) / DSP_WAVES;
   return g < DSP_GRID ? g : DSP_GRID;
+}
+
+// Workgroups of a launch: as many as the registers of the rank's kernel let reside together.
+int dsp_launch(int64_t v, int64_t rank) {
+  const int64_t g = dsp_nwg(v), most = rank <= 128 ? DSP_GRID : 512;
+  return g < most ? (int)g : (int)most;
 }
 
 }  // namespace
@@ -279,18 +433,17 @@ SV_API int snowllm_dspark_markov(const void* base, const void* w1, const void* w
   DspArgs a{(const float*)base, (const uint16_t*)w1, (const uint16_t*)w2, anchor,
             (const uint16_t*)pre_head, conf_weight, conf_bias, out, confidence,
             (uint64_t*)workspace, v, base_stride, ps, (int)b, (int)rank, (int)block,
-            confidence ? (int)h : 0, (int)dsp_nwg(v), fp32_bias != 0, 0};
+            confidence ? (int)h : 0, dsp_launch(v, rank), fp32_bias != 0, 0};
   for (int j = 0; j < block; ++j) {
     a.j = j;
-    if (b == 1)
-      hipLaunchKernelGGL(dsp_markov_kernel<1>, dim3((unsigned)a.nwg), dim3(DSP_NT), 0,
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)(a.nwg + (confidence ? 1 : 0))), dim3(DSP_NT), 0,
                          (hipStream_t)stream, a);
-    else if (b <= 4)
-      hipLaunchKernelGGL(dsp_markov_kernel<4>, dim3((unsigned)a.nwg), dim3(DSP_NT), 0,
-                         (hipStream_t)stream, a);
-    else
-      hipLaunchKernelGGL(dsp_markov_kernel<DSP_MAX_B>, dim3((unsigned)a.nwg), dim3(DSP_NT), 0,
-                         (hipStream_t)stream, a);
+    };
+    if (rank <= 64) go(dsp_markov_kernel<2>);
+    else if (rank <= 128) go(dsp_markov_kernel<4>);
+    else if (rank <= 256) go(dsp_markov_kernel<8>);
+    else go(dsp_markov_kernel<16>);
     SV_CHECK_LAUNCH();
   }
   return SV_OK;

@@ -68,6 +68,40 @@ def test_markov_equals_oracle(gpu, V, rank, b, block, pad, fp32):
         assert path[1, 1].item() == 0 and 10 <= path[1, 2].item() < 20
 
 
+@pytest.mark.parametrize("kind", ["plain", "-inf", "lowest", "equal", "zeros", "infinite", "tiny"])
+@pytest.mark.parametrize("V,rank,b", [(77, 8, 16), (9000, 72, 5), (1290, 264, 3)])
+def test_markov_bounds_keep_the_pick(gpu, V, rank, b, kind):
+    """Ranks and vocabularies off the tile sizes, and rows whose bounds say little: masked logits,
+    equal scores (more candidates than a workgroup keeps), infinities, values below the normal
+    range. The picks are the fp64 oracle's, bit for bit."""
+    from snowllm_amd.draft_heads import MarkovHead
+    _say(f"dspark markov bounds V={V} rank={rank} b={b} {kind}")
+    block = 3
+    W1, W2, base, anchor, *_ = _markov_case(V, rank, b, block, V + rank)
+    if kind in ("-inf", "lowest"):
+        low = float("-inf") if kind == "-inf" else torch.finfo(torch.float32).min
+        base[:, :-3] = low
+        base[1] = low                           # a row with nothing left
+    elif kind == "equal":
+        W2[:] = W2[0].clone()
+        base[:] = 1.5
+    elif kind == "zeros":
+        W1.zero_(), base.zero_()
+    elif kind == "infinite":
+        W2[5, 1], W2[9, 3], base[0, 4], base[2, 6] = float("inf"), float("nan"), float("inf"), float("nan")
+    elif kind == "tiny":
+        W1[:], base[:] = W1 * 2.0 ** -133, base * 2.0 ** -20
+        W2[:] = W2 * 2.0 ** 110
+    head = MarkovHead(W1.cuda(), W2.cuda())
+    path = torch.full((b, block), -7, dtype=torch.int64, device="cuda")
+    head.propose(None, base.cuda(), anchor.cuda(), path)
+    torch.cuda.synchronize()
+    with np.errstate(all="ignore"):
+        want = D.markov(base.numpy(), _bits(W1), _bits(W2), anchor.numpy(), block)
+    want = want[0] if isinstance(want, tuple) else want
+    assert np.array_equal(path.cpu().numpy(), want)
+
+
 def test_markov_without_confidence_and_graph_replay(gpu):
     """No confidence output; the arrival counter carries across captured replays."""
     from snowllm_amd.draft_heads import MarkovHead
