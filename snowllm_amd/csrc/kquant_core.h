@@ -240,9 +240,6 @@ __device__ __forceinline__ float byte_f(uint32_t w, int i) {
   return (float)((w >> (8 * i)) & 0xffu);
 }
 
-// One 16-column x 256-weight tile. Returns the superblock's contribution in the C layout
-// (column lane & 15, rows 4*(lane >> 4) + i), still in units of the operand scaling.
-// xa: A operands of the 8 sub-blocks, sx0/sx1: negated sub-block sums (f32 MFMA A operand).
 // Q5_K: the fifth bit of sub-block j's weights, placed on the 16-bit lanes of q4_group's four
 // words (bytes (0, 2), (1, 3) of qa and of qb), at bit `at` (4: low nibbles, 8: high nibbles,
 // which q4_group leaves at 16 q).
@@ -264,145 +261,159 @@ __device__ __forceinline__ half8 or_half8(half8 v, const uint32_t (&e)[4]) {
 
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 
-// Q6_K: the exact fp16 values q - 32 of one 32-weight run in kperm slot order, from its ql
-// words (wa, wb: bytes l = 8 kq .. 8 kq + 7), the nibble shift (0 low, 4 high) and its qh words
-// (ha, hb) with the run's bit pair at hs.
-__device__ __forceinline__ half8 q6_run(uint32_t wa, uint32_t wb, uint32_t ha, uint32_t hb, int sh,
-                                        int hs, uint32_t M) {
-  const uint32_t w0 = and_or((wa >> sh) & 0x000f000fu, 0xffffffffu, ((ha >> hs) & 0x00030003u) << 4);
-  const uint32_t w1 = and_or((wa >> (8 + sh)) & 0x000f000fu, 0xffffffffu,
-                             ((ha >> (8 + hs)) & 0x00030003u) << 4);
-  const uint32_t w2 = and_or((wb >> sh) & 0x000f000fu, 0xffffffffu, ((hb >> hs) & 0x00030003u) << 4);
-  const uint32_t w3 = and_or((wb >> (8 + sh)) & 0x000f000fu, 0xffffffffu,
-                             ((hb >> (8 + hs)) & 0x00030003u) << 4);
-  // 0x6400 | q = 1024 + q exactly; minus 1056 gives q - 32 exactly
-  const half2v off = {(_Float16)1056.0f, (_Float16)1056.0f};
-  const half2v v0 = __builtin_bit_cast(half2v, w0 | M) - off;
-  const half2v v1 = __builtin_bit_cast(half2v, w1 | M) - off;
-  const half2v v2 = __builtin_bit_cast(half2v, w2 | M) - off;
-  const half2v v3 = __builtin_bit_cast(half2v, w3 | M) - off;
-  return as_half8(__builtin_bit_cast(uint32_t, v0), __builtin_bit_cast(uint32_t, v1),
-                  __builtin_bit_cast(uint32_t, v2), __builtin_bit_cast(uint32_t, v3));
+// Four Q6_K quants of one 32-weight run as bytes: run p of a half takes the low (p < 2) or high
+// nibbles of its ql word and bit pair p of its qh word.
+__device__ __forceinline__ uint32_t q6_bytes(uint32_t wl, uint32_t wh, int p) {
+  const uint32_t lo = (p < 2 ? wl : wl >> 4) & 0x0f0f0f0fu;
+  const uint32_t hi = p == 0 ? wh << 4 : p == 1 ? wh << 2 : p == 2 ? wh : wh >> 2;
+  return and_or(hi, 0x30303030u, lo);
 }
 
-__device__ __forceinline__ float sbyte_f(uint32_t w, int i) {
-  return (float)(int8_t)((w >> (8 * i)) & 0xffu);
+__device__ __forceinline__ half2v half2_of(uint32_t w) { return __builtin_bit_cast(half2v, w); }
+
+// One 16-column x 256-weight tile against MT row tiles: out[m] is the superblock's contribution
+// in the C layout (column lane & 15, rows 4*(lane >> 4) + i), still in units of the operand
+// scaling. x(m, j): A operand of row tile m's sub-block j; sx0/sx1: negated sub-block sums (f32
+// MFMA A operand). Each sub-block is decoded once and multiplied with every row tile, and a row
+// tile's products and sums do not depend on MT: every width gives a row the same bits.
+template <int FMT, int MT, class X>
+__device__ __forceinline__ void tile_superblock_rows(const u32x4* qv, u32x4 meta, uint32_t dq,
+                                                     X&& x, const float* sx0, const float* sx1,
+                                                     int kq, uint32_t M, floatx4 (&out)[MT]) {
+  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+  if constexpr (FMT == FMT_Q6_K) {
+    // w = d sc_g (q - 32) with a scale per 16 weights: a lane's 8 weights of a 32-weight run lie
+    // in one group (kq < 2: the first), so its scale goes into the operand. sc (q - 32) does not
+    // fit fp16's 11 bits, so sc = 16 sh + sl (sl in [-8, 7], sh in [-8, 8]) and the integers
+    // sh (q - 32) and sl (q - 32), both exact, are multiplied separately: (1024 + q) s - 1056 s
+    // is one fused multiply-add whose result fits. All sums of the superblock stay in the matrix
+    // cores' fp32 accumulators; d is applied once. Per 32-weight run about 25 vector
+    // instructions for any number of rows; with a product per scale and lane-masked operands it
+    // was 56, 8 of them per row tile, and the vector units were what bound Q6_K. MI355X, us,
+    // before -> now: 151,936 x 2048 at 9 rows 103 -> 90, 4096 x 14,336 at 126 rows 79 -> 62,
+    // 14,336 x 4096 at 9 rows 29 -> 25; Q6_K experts, 60 rows, 189 -> 169.
+    const float d = f16_to_f32((uint16_t)((threadIdx.x & 1) ? (dq >> 16) : (dq & 0xffff)));
+    const int sel = kq < 2 ? 0 : 8;
+    const uint32_t sw[4] = {meta.x >> sel, meta.y >> sel, meta.z >> sel, meta.w >> sel};
+    const half2v off = {(_Float16)1032.0f, (_Float16)1032.0f};
+    const half2v bias = {(_Float16)-1056.0f, (_Float16)-1056.0f};
+    floatx4 hi[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) hi[m] = out[m] = zero;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int n = j >> 2, p = j & 3;
+      // sc + 136 of runs 2 (p / 2) (low half) and 2 (p / 2) + 1
+      const uint32_t u = ((sw[j >> 1] & 0x00ff00ffu) ^ 0x00800080u) + 0x00080008u;
+      const half2v sl = half2_of(and_or(u, 0x000f000fu, M)) - off;
+      const half2v sh = half2_of(and_or(u >> 4, 0x001f001fu, M)) - off;
+      const half2v bl = sl * bias, bh = sh * bias;
+      const half2v l = {sl[p & 1], sl[p & 1]}, h = {sh[p & 1], sh[p & 1]};
+      const half2v lb = {bl[p & 1], bl[p & 1]}, hb = {bh[p & 1], bh[p & 1]};
+      const u32x4 ql = qv[n];
+      const uint32_t wa = q6_bytes((p & 1) ? ql.z : ql.x, n ? qv[2].z : qv[2].x, p);
+      const uint32_t wb = q6_bytes((p & 1) ? ql.w : ql.y, n ? qv[2].w : qv[2].y, p);
+      // bytes (0, 2) and (1, 3) under the exponent byte 0x64: 1024 + q
+      const half2v v[4] = {half2_of(__builtin_amdgcn_perm(M, wa, 0x05020500u)),
+                           half2_of(__builtin_amdgcn_perm(M, wa, 0x05030501u)),
+                           half2_of(__builtin_amdgcn_perm(M, wb, 0x05020500u)),
+                           half2_of(__builtin_amdgcn_perm(M, wb, 0x05030501u))};
+      uint32_t wl[4], wh[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        wl[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(v[i], l, lb));
+        wh[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(v[i], h, hb));
+      }
+      const half8 b_lo = as_half8(wl[0], wl[1], wl[2], wl[3]);
+      const half8 b_hi = as_half8(wh[0], wh[1], wh[2], wh[3]);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const half8 xa = x(m, j);
+        out[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa, b_lo, out[m], 0, 0, 0);
+        hi[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa, b_hi, hi[m], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) out[m][i] = d * __builtin_fmaf(16.0f, hi[m][i], out[m][i]);
+  } else {
+    float beta_lo, beta_hi;  // beta for sub-blocks kq and kq + 4
+#pragma unroll
+    for (int m = 0; m < MT; ++m) out[m] = zero;
+    auto apply = [&](int j, float aj, half8 b) {
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const floatx4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(x(m, j), b, zero, 0, 0, 0);
+        out[m] += aj * c;
+      }
+    };
+    if constexpr (FMT == FMT_Q4_K || FMT == FMT_Q5_K) {
+      const float d = f16_to_f32((uint16_t)(meta.x & 0xffff));
+      const float dmin = f16_to_f32((uint16_t)(meta.x >> 16));
+      const uint32_t s0 = meta.y, s1 = meta.z, s2 = meta.w;
+      const uint32_t sc03 = s0 & 0x3f3f3f3fu;
+      const uint32_t m03 = s1 & 0x3f3f3f3fu;
+      const uint32_t sc47 = (s2 & 0x0f0f0f0fu) | ((s0 >> 2) & 0x30303030u);
+      const uint32_t m47 = ((s2 >> 4) & 0x0f0f0f0fu) | ((s1 >> 2) & 0x30303030u);
+      float a[8];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        a[i] = d * byte_f(sc03, i);
+        a[4 + i] = d * byte_f(sc47, i);
+      }
+      const float m_lo = dmin * byte_f(m03, kq);
+      const float m_hi = dmin * byte_f(m47, kq);
+      // even sub-blocks carry the 1024 offset; odd ones read 1024 + 16 q, i.e. 64 after the 1/16
+      const float off = (kq & 1) ? 64.0f : 1024.0f;
+      beta_lo = __builtin_fmaf(off, d * byte_f(sc03, kq), m_lo);  // a[kq] without a select chain
+      beta_hi = __builtin_fmaf(off, d * byte_f(sc47, kq), m_hi);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const u32x4 q = qv[g >> 1];
+        half8 lo, hi;
+        q4_group((g & 1) ? q.z : q.x, (g & 1) ? q.w : q.y, M, lo, hi);
+        if constexpr (FMT == FMT_Q5_K) {
+          // the fifth bits into the nibble lanes (bit 4 of 1024 + q, bit 8 of 1024 + 16 q)
+          uint32_t e[4];
+          q5_bits(qv[2].x, qv[2].y, 2 * g, 4, e);
+          lo = or_half8(lo, e);
+          q5_bits(qv[2].x, qv[2].y, 2 * g + 1, 8, e);
+          hi = or_half8(hi, e);
+        }
+        apply(2 * g, a[2 * g], lo);
+        apply(2 * g + 1, a[2 * g + 1] * 0.0625f, hi);
+      }
+    } else {
+      const uint32_t dw[4] = {meta.x, meta.y, meta.z, meta.w};
+      // a[kq], a[4 + kq] read straight from the packed scales (no select chain on kq)
+      beta_lo = 1152.0f * f16_to_f32((uint16_t)(((kq & 1) ? (dw[kq >> 1] >> 16) : dw[kq >> 1]) & 0xffff));
+      beta_hi = 1152.0f * f16_to_f32((uint16_t)(((kq & 1) ? (dw[2 + (kq >> 1)] >> 16) : dw[2 + (kq >> 1)]) & 0xffff));
+#pragma unroll
+      for (int jp = 0; jp < 4; ++jp) {
+        const u32x4 q = qv[jp];
+        apply(2 * jp, f16_to_f32((uint16_t)(dw[jp] & 0xffff)), q8_sub(q.x, q.y, M));
+        apply(2 * jp + 1, f16_to_f32((uint16_t)(dw[jp] >> 16)), q8_sub(q.z, q.w, M));
+      }
+    }
+    // offset/min term: acc += (-Sx) * beta over the 8 sub-blocks (k = lane >> 4 in each half)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      out[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(sx0[m], beta_lo, out[m], 0, 0, 0);
+      out[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(sx1[m], beta_hi, out[m], 0, 0, 0);
+    }
+  }
 }
 
+// One row tile.
 template <int FMT>
 __device__ __forceinline__ floatx4 tile_superblock(const u32x4* qv, u32x4 meta, uint32_t dq,
                                                    const half8* xa, float sx0, float sx1, int kq,
                                                    uint32_t M) {
-  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
-  floatx4 acc = zero;
-  float a[8];
-  float beta_lo, beta_hi;  // beta for sub-blocks kq and kq + 4
-  if constexpr (FMT == FMT_Q6_K) {
-    // w = d sc_g (q - 32) with a scale per 16 weights: each 32-weight run is multiplied twice,
-    // once with the B lanes of its first 16 weights (kq < 2) and once with the rest, each
-    // product scaled by its own sc; q - 32 is exact in fp16, so no offset term is needed
-    const float d = f16_to_f32((uint16_t)((threadIdx.x & 1) ? (dq >> 16) : (dq & 0xffff)));
-    const uint32_t keep_lo = kq < 2 ? 0xffffffffu : 0u, keep_hi = ~keep_lo;
-    const uint32_t sw[4] = {meta.x, meta.y, meta.z, meta.w};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int n = j >> 2, p = j & 3;
-      const u32x4 ql = qv[n];
-      const uint32_t wa = (p & 1) ? ql.z : ql.x, wb = (p & 1) ? ql.w : ql.y;
-      const uint32_t ha = n ? qv[2].z : qv[2].x, hb = n ? qv[2].w : qv[2].y;
-      const half8 b = q6_run(wa, wb, ha, hb, (p >> 1) * 4, 2 * p, M);
-      const u32x4 bw = __builtin_bit_cast(u32x4, b);
-      const half8 b_lo = __builtin_bit_cast(half8, bw & keep_lo);
-      const half8 b_hi = __builtin_bit_cast(half8, bw & keep_hi);
-      const int si = 8 * n + 2 * p;  // scales of weights l < 16 and l >= 16
-      const float s_lo = d * sbyte_f(sw[si >> 2], si & 3);
-      const float s_hi = d * sbyte_f(sw[(si + 1) >> 2], (si + 1) & 3);
-      floatx4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[j], b_lo, zero, 0, 0, 0);
-      acc += s_lo * c;
-      c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[j], b_hi, zero, 0, 0, 0);
-      acc += s_hi * c;
-    }
-    return acc;
-  } else if constexpr (FMT == FMT_Q4_K || FMT == FMT_Q5_K) {
-    const float d = f16_to_f32((uint16_t)(meta.x & 0xffff));
-    const float dmin = f16_to_f32((uint16_t)(meta.x >> 16));
-    const uint32_t s0 = meta.y, s1 = meta.z, s2 = meta.w;
-    const uint32_t sc03 = s0 & 0x3f3f3f3fu;
-    const uint32_t m03 = s1 & 0x3f3f3f3fu;
-    const uint32_t sc47 = (s2 & 0x0f0f0f0fu) | ((s0 >> 2) & 0x30303030u);
-    const uint32_t m47 = ((s2 >> 4) & 0x0f0f0f0fu) | ((s1 >> 2) & 0x30303030u);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      a[i] = d * byte_f(sc03, i);
-      a[4 + i] = d * byte_f(sc47, i);
-    }
-    const float m_lo = dmin * byte_f(m03, kq);
-    const float m_hi = dmin * byte_f(m47, kq);
-    // even sub-blocks carry the 1024 offset; odd ones read 1024 + 16 q, i.e. 64 after the 1/16
-    const float off = (kq & 1) ? 64.0f : 1024.0f;
-    beta_lo = __builtin_fmaf(off, d * byte_f(sc03, kq), m_lo);  // a[kq] without a select chain
-    beta_hi = __builtin_fmaf(off, d * byte_f(sc47, kq), m_hi);
-    const u32x4 q0 = qv[0], q1 = qv[1];
-    half8 lo, hi;
-    floatx4 c;
-    // Q5_K: OR the fifth bits into the nibble lanes (bit 4 of 1024 + q, bit 8 of 1024 + 16 q)
-    auto fifth = [&](int j, half8& l, half8& h) {
-      if constexpr (FMT == FMT_Q5_K) {
-        uint32_t e[4];
-        q5_bits(qv[2].x, qv[2].y, j, 4, e);
-        l = or_half8(l, e);
-        q5_bits(qv[2].x, qv[2].y, j + 1, 8, e);
-        h = or_half8(h, e);
-      }
-    };
-    q4_group(q0.x, q0.y, M, lo, hi);
-    fifth(0, lo, hi);
-    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[0], lo, zero, 0, 0, 0);
-    acc += a[0] * c;
-    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[1], hi, zero, 0, 0, 0);
-    acc += (a[1] * 0.0625f) * c;
-    q4_group(q0.z, q0.w, M, lo, hi);
-    fifth(2, lo, hi);
-    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[2], lo, zero, 0, 0, 0);
-    acc += a[2] * c;
-    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[3], hi, zero, 0, 0, 0);
-    acc += (a[3] * 0.0625f) * c;
-    q4_group(q1.x, q1.y, M, lo, hi);
-    fifth(4, lo, hi);
-    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[4], lo, zero, 0, 0, 0);
-    acc += a[4] * c;
-    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[5], hi, zero, 0, 0, 0);
-    acc += (a[5] * 0.0625f) * c;
-    q4_group(q1.z, q1.w, M, lo, hi);
-    fifth(6, lo, hi);
-    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[6], lo, zero, 0, 0, 0);
-    acc += a[6] * c;
-    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[7], hi, zero, 0, 0, 0);
-    acc += (a[7] * 0.0625f) * c;
-  } else {
-    const uint32_t dw[4] = {meta.x, meta.y, meta.z, meta.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      a[2 * i] = f16_to_f32((uint16_t)(dw[i] & 0xffff));
-      a[2 * i + 1] = f16_to_f32((uint16_t)(dw[i] >> 16));
-    }
-    // a[kq], a[4 + kq] read straight from the packed scales (no select chain on kq)
-    beta_lo = 1152.0f * f16_to_f32((uint16_t)(((kq & 1) ? (dw[kq >> 1] >> 16) : dw[kq >> 1]) & 0xffff));
-    beta_hi = 1152.0f * f16_to_f32((uint16_t)(((kq & 1) ? (dw[2 + (kq >> 1)] >> 16) : dw[2 + (kq >> 1)]) & 0xffff));
-#pragma unroll
-    for (int jp = 0; jp < 4; ++jp) {
-      const u32x4 q = qv[jp];
-      floatx4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[2 * jp], q8_sub(q.x, q.y, M), zero, 0,
-                                                          0, 0);
-      acc += a[2 * jp] * c;
-      c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[2 * jp + 1], q8_sub(q.z, q.w, M), zero, 0, 0, 0);
-      acc += a[2 * jp + 1] * c;
-    }
-  }
-  // offset/min term: acc += (-Sx) * beta over the 8 sub-blocks (k = lane >> 4 in each half)
-  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sx0, beta_lo, acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sx1, beta_hi, acc, 0, 0, 0);
-  return acc;
+  floatx4 out[1];
+  tile_superblock_rows<FMT, 1>(qv, meta, dq, [&](int, int j) { return xa[j]; }, &sx0, &sx1, kq, M,
+                               out);
+  return out[0];
 }
 
 // Repacked weight layout per 16-column tile and superblock ("tile-superblock", ts):

@@ -1,5 +1,6 @@
 """GPU kernels over more than 16 rows at the edges of their tiles and dispatch rules: the bits of
 the 16-row launches and the fp64 product."""
+import numpy as np
 import pytest
 import torch
 
@@ -38,3 +39,27 @@ def test_dense_gemv_wide_edges(gpu, wt, M, N, K):
     assert torch.equal(out, tiles)
     # exact products summed in 32 bits: K roundings of 2^-24 at most
     assert rel(out.cpu(), x.double().cpu() @ w.double().cpu().T) < K * 2.0 ** -24
+
+
+@pytest.mark.parametrize("m", [16, 33])
+def test_q6k_every_scale_is_exact(gpu, m):
+    """Q6_K scales over the whole of int8 against quants 0, 63 and random ones: rows with a single
+    1 read single weights d sc (q - 32), whose integer part is exact, so one rounding is left."""
+    from oracle import quant as Q
+    from snowllm_amd import ops
+    n, k = 64, 1024
+    print(f"q6k scales m={m}", flush=True)
+    raw = Q.make_q6_k(n, k, seed=m)
+    b = raw.reshape(-1, 210)
+    b[:, 192:208] = np.arange(b.shape[0] * 16, dtype=np.uint8).reshape(-1, 16)
+    b[0::3, :192], b[1::3, :192] = 0x00, 0xff
+    x = torch.zeros(m, k)
+    at = (torch.arange(m) * 37) % k
+    x[torch.arange(m), at] = 1.0
+    quant, meta = ops.gemm_kquant_shuffle_b(6, torch.from_numpy(raw).cuda(), n, k)
+    ws = torch.empty(ops.gemm_kquant_a_ws_bytes(m, k), dtype=torch.uint8, device="cuda")
+    out = torch.empty(m, n, device="cuda")
+    ops.gemm_kquant_a(6, x.bfloat16().cuda(), quant, meta, out, m, n, k, ws)
+    torch.cuda.synchronize()
+    want = torch.from_numpy(Q.dequant(raw, 6, n, k)).double()[:, at].T
+    assert ((out.cpu().double() - want).abs() <= want.abs() * 2.0 ** -23).all()
