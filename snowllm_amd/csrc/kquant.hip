@@ -87,81 +87,16 @@ __global__ void __launch_bounds__(NW * 64) kquant_gemv(const u32x4* __restrict__
 }
 
 // ---------------------------------------------------------------------------------------
-// The same GEMV over MT 16-row tiles at once (a verify step wider than 16 rows): each wave
-// loads a superblock's weights once, decodes them once into the fp16 B operands, and multiplies
-// them against the prepared operands of every row tile (blockIdx.y: the group of MT tiles).
-// The per-row arithmetic and the waves' superblock split are those of kquant_gemv with NW
-// waves, so every row gets the bits of the 16-row launch.
+// The same GEMV over MT 16-row tiles at once (a verify step wider than 16 rows; blockIdx.y: the
+// group of MT tiles): each wave decodes a superblock of NT column tiles once for the prepared
+// operands of MT row tiles, and the next superblock's operands load into the registers that the
+// current one's products free. Bound: the L2 reads (26 KB per 2 x 4 tiles and superblock, 13 KB
+// per 1 x 2) and the vector units' decode and rescaling, both shared by more tiles the more a
+// wave holds; the registers of two waves per SIMD limit that to 2 x 4. Q4_K 4096 x 14336, 126
+// rows: 50 -> 37 us against one row tile by two column tiles with no load ahead. The per-row arithmetic and the waves' superblock split are those of
+// kquant_gemv with NW waves, so every row gets the bits of the 16-row launch.
 // ---------------------------------------------------------------------------------------
-template <int FMT>
-struct DecodedSb {
-  half8 b[8];     // B operands of the 8 sub-blocks
-  float a[8];     // per-sub-block scales (odd Q4_K sub-blocks: x 1/16 for the 16 q encoding)
-  float beta_lo, beta_hi;
-};
-
-template <int FMT>
-__device__ __forceinline__ void decode_sb(const u32x4* qv, u32x4 meta, int kq, uint32_t M,
-                                          DecodedSb<FMT>& d) {
-  if constexpr (FMT == FMT_Q4_K) {
-    const float dd = f16_to_f32((uint16_t)(meta.x & 0xffff));
-    const float dmin = f16_to_f32((uint16_t)(meta.x >> 16));
-    const uint32_t s0 = meta.y, s1 = meta.z, s2 = meta.w;
-    const uint32_t sc03 = s0 & 0x3f3f3f3fu;
-    const uint32_t m03 = s1 & 0x3f3f3f3fu;
-    const uint32_t sc47 = (s2 & 0x0f0f0f0fu) | ((s0 >> 2) & 0x30303030u);
-    const uint32_t m47 = ((s2 >> 4) & 0x0f0f0f0fu) | ((s1 >> 2) & 0x30303030u);
-    float a[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      a[i] = dd * byte_f(sc03, i);
-      a[4 + i] = dd * byte_f(sc47, i);
-    }
-    const float m_lo = dmin * byte_f(m03, kq);
-    const float m_hi = dmin * byte_f(m47, kq);
-    const float off = (kq & 1) ? 64.0f : 1024.0f;
-    d.beta_lo = __builtin_fmaf(off, dd * byte_f(sc03, kq), m_lo);
-    d.beta_hi = __builtin_fmaf(off, dd * byte_f(sc47, kq), m_hi);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) d.a[j] = (j & 1) ? a[j] * 0.0625f : a[j];
-    q4_group(qv[0].x, qv[0].y, M, d.b[0], d.b[1]);
-    q4_group(qv[0].z, qv[0].w, M, d.b[2], d.b[3]);
-    q4_group(qv[1].x, qv[1].y, M, d.b[4], d.b[5]);
-    q4_group(qv[1].z, qv[1].w, M, d.b[6], d.b[7]);
-  } else {
-    const uint32_t dw[4] = {meta.x, meta.y, meta.z, meta.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      d.a[2 * i] = f16_to_f32((uint16_t)(dw[i] & 0xffff));
-      d.a[2 * i + 1] = f16_to_f32((uint16_t)(dw[i] >> 16));
-    }
-    d.beta_lo = 1152.0f * f16_to_f32((uint16_t)(((kq & 1) ? (dw[kq >> 1] >> 16) : dw[kq >> 1]) & 0xffff));
-    d.beta_hi = 1152.0f * f16_to_f32((uint16_t)(((kq & 1) ? (dw[2 + (kq >> 1)] >> 16) : dw[2 + (kq >> 1)]) & 0xffff));
-#pragma unroll
-    for (int jp = 0; jp < 4; ++jp) {
-      d.b[2 * jp] = q8_sub(qv[jp].x, qv[jp].y, M);
-      d.b[2 * jp + 1] = q8_sub(qv[jp].z, qv[jp].w, M);
-    }
-  }
-}
-
-// tile_superblock's arithmetic on decoded weights: the same products and sums in the same order.
-template <int FMT>
-__device__ __forceinline__ floatx4 apply_sb(const DecodedSb<FMT>& d, const half8* xa, float sx0,
-                                            float sx1) {
-  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
-  floatx4 acc = zero;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const floatx4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[j], d.b[j], zero, 0, 0, 0);
-    acc += d.a[j] * c;
-  }
-  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sx0, d.beta_lo, acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sx1, d.beta_hi, acc, 0, 0, 0);
-  return acc;
-}
-
-template <int FMT, int NW, int MT, int NT = 1>
+template <int FMT, int NW, int MT, int NT>
 __global__ void __launch_bounds__(NW * 64) kquant_gemv_mt(const u32x4* __restrict__ quant,
                                                           const u32x4* __restrict__ meta,
                                                           const void* __restrict__ ws,
@@ -177,13 +112,14 @@ __global__ void __launch_bounds__(NW * 64) kquant_gemv_mt(const u32x4* __restric
   const int tile0 = blockIdx.x * NT;  // NT column tiles share each row tile's operands
   const int m0 = blockIdx.y * MT;
   const int row_tiles = (M + TILE_M - 1) / TILE_M;
-  const int mt = row_tiles - m0 < MT ? row_tiles - m0 : MT;
   const GemvStreams st = make_streams<FMT>(quant, meta, ws, tiles, S, lane, 16);
   __amdgpu_buffer_rsrc_t xr[MT], sxr[MT], scr[MT];
   uint32_t vx[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
-    XPrepView xv = xprep_view((char*)ws + (size_t)(m0 + m) * tile_bytes, S);
+    // a row tile past the last: the last one's sums and scales, and no operands
+    const int tile = m0 + m < row_tiles ? m0 + m : row_tiles - 1;
+    XPrepView xv = xprep_view((char*)ws + (size_t)tile * tile_bytes, S);
     xr[m] = __builtin_amdgcn_make_buffer_rsrc((void*)xv.xop, 0, S * 8 * 64 * 16, 0x00020000);
     sxr[m] = __builtin_amdgcn_make_buffer_rsrc((void*)xv.sxop, 0, S * 2 * 64 * 4, 0x00020000);
     scr[m] = __builtin_amdgcn_make_buffer_rsrc((void*)xv.scale, 0, S * 16 * 4, 0x00020000);
@@ -195,60 +131,62 @@ __global__ void __launch_bounds__(NW * 64) kquant_gemv_mt(const u32x4* __restric
   for (int m = 0; m < MT; ++m)
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[m][t] = floatx4{0.f, 0.f, 0.f, 0.f};
-  for (int s = w; s < S; s += NW) {
-    // (a tile past the last reads nothing: its buffer offsets are out of range)
-    u32x4 q[NT][QV], mt4[NT];
-    uint32_t dq[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) dq[t] = 0u;
-    load_sb_w<FMT, NT>(q, mt4, st, s, S, tile0, 1);
-    if constexpr (FMT == FMT_Q6_K) load_sb_d<NT>(dq, st, s, S, tile0, 1);
-    // every row tile's operands of this superblock in flight with the weights
-    u32x4 x[MT][8];
-    float sx0[MT], sx1[MT];
-    floatx4 sc[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      if (m >= mt) break;  // uniform
-#pragma unroll
-      for (int j = 0; j < 8; ++j) x[m][j] = bload4(xr[m], vx[m], (uint32_t)((s * 8 + j) * 64 * 16));
-      sx0[m] = bload1(sxr[m], lane * 4, (uint32_t)((s * 2 + 0) * 64 * 4));
-      sx1[m] = bload1(sxr[m], lane * 4, (uint32_t)((s * 2 + 1) * 64 * 4));
-      sc[m] = __builtin_bit_cast(floatx4, bload4(scr[m], kq * 16, (uint32_t)(s * 16 * 4)));
-    }
+  // the operands of one superblock; the next one's go into the same registers as they fall free
+  // (a tile past the last column reads nothing: its buffer offsets are out of range)
+  u32x4 q[NT][1][QV], mt4[NT][1], x[MT][8];
+  uint32_t dq[NT][1];
+  float sx0[MT], sx1[MT];
+  floatx4 sc[MT];
+  auto load_w = [&](int t, int s) {
+    load_sb_w<FMT, 1>(q[t], mt4[t], st, s, S, tile0 + t, 1);
+    if constexpr (FMT == FMT_Q6_K) load_sb_d<1>(dq[t], st, s, S, tile0 + t, 1);
+    else dq[t][0] = 0u;
+  };
+  auto load_x = [&](int m, int j, int s) {
+    x[m][j] = bload4(xr[m], vx[m], (uint32_t)((s * 8 + j) * 64 * 16));
+  };
+  auto load_sx = [&](int m, int s) {
+    sx0[m] = bload1(sxr[m], lane * 4, (uint32_t)((s * 2 + 0) * 64 * 4));
+    sx1[m] = bload1(sxr[m], lane * 4, (uint32_t)((s * 2 + 1) * 64 * 4));
+    sc[m] = __builtin_bit_cast(floatx4, bload4(scr[m], kq * 16, (uint32_t)(s * 16 * 4)));
+  };
+  auto step = [&](int s, auto more) {
+    constexpr bool MORE = decltype(more)::value;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      if constexpr (FMT == FMT_Q4_K || FMT == FMT_Q8_0) {
-        DecodedSb<FMT> d;
-        decode_sb<FMT>(q[t], mt4[t], kq, Mv, d);
+      floatx4 sb[MT];
+      tile_superblock_rows<FMT, MT>(
+          q[t][0], mt4[t][0], dq[t][0],
+          [&](int m, int j) {
+            const half8 v = __builtin_bit_cast(half8, x[m][j]);
+            if (MORE && t == NT - 1) load_x(m, j, s + NW);
+            return v;
+          },
+          sx0, sx1, kq, Mv, sb);
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-          if (m >= mt) break;  // uniform
-          half8 xa[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) xa[j] = __builtin_bit_cast(half8, x[m][j]);
-          const floatx4 sb = apply_sb<FMT>(d, xa, sx0[m], sx1[m]);
-          acc[m][t] += sb * sc[m];
-        }
-      } else {
-        // Q5_K / Q6_K: the weights loaded once, decoded again for each row tile by the 16-row
-        // kernel's own routine (their decoded operands do not fit the registers of four tiles)
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-          if (m >= mt) break;  // uniform
-          half8 xa[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) xa[j] = __builtin_bit_cast(half8, x[m][j]);
-          const floatx4 sb =
-              tile_superblock<FMT>(q[t], mt4[t], dq[t], xa, sx0[m], sx1[m], kq, Mv);
-          acc[m][t] += sb * sc[m];
-        }
-      }
+      for (int m = 0; m < MT; ++m) acc[m][t] += sb[m] * sc[m];
+      if (MORE) load_w(t, s + NW);
     }
+    if (MORE)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) load_sx(m, s + NW);
+  };
+  if (w < S) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) load_w(t, w);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) load_x(m, j, w);
+      load_sx(m, w);
+    }
+    int s = w;
+    for (; s + NW < S; s += NW) step(s, std::true_type{});
+    step(s, std::false_type{});
   }
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
-    if (m >= mt) break;  // uniform
+    if (m0 + m >= row_tiles) break;  // uniform
     if (m) __syncthreads();
     combine_waves<NT, NW>(part, acc[m], w, lane);
     for (int idx = threadIdx.x; idx < NT * 64; idx += NW * 64) {
@@ -277,22 +215,47 @@ int launch_gemv_mt(const void* quant, const void* meta, const void* ws, void* c,
   const int tiles = N / TILE_N;
   const int row_tiles = (M + TILE_M - 1) / TILE_M;
   const size_t tb = xprep_tile_bytes(S);
-  // One row tile per workgroup (blockIdx.y), two column tiles per workgroup where that still
-  // leaves 192 or more workgroups. Measured on MI355X (prepared operands, the weights from
-  // HBM): decoding a weight superblock once for several row tiles saves less than the
-  // workgroups it takes away. N = 2048, K = 4096 at 36 / 54 / 128 rows: 9.3 / 11.2 / 11.6 us
-  // with three or four row tiles per workgroup against 6.0 / 6.1 / 8.6 us; N = 5120, K = 2048
-  // at 128 rows 20.8 against 11.1 us; N = 14336, K = 4096 at 72 rows 42.8 against 30.4 us.
-  // One column tile only wins at N = 2048 and 18 rows (4.9 against 6.0 us). The same bits
-  // either way (every row gets the 16-row launch's arithmetic).
-  const int nt = (int64_t)(tiles / 2) * row_tiles >= 192 ? 2 : 1;
   auto go = [&](auto kern, int mt, int ntile) {
     hipLaunchKernelGGL(kern, dim3((tiles + ntile - 1) / ntile, (row_tiles + mt - 1) / mt),
                        dim3(NW * 64), 0, s, (const u32x4*)quant, (const u32x4*)meta, ws, c, M,
                        N, S, c_bf16, tb, ldc);
   };
-  if (nt == 2) go(kquant_gemv_mt<FMT, NW, 1, 2>, 1, 2);
-  else go(kquant_gemv_mt<FMT, NW, 1>, 1, 1);
+  // Two row tiles by four (or two) column tiles where such workgroups, one to a CU, fill the 256
+  // CUs' last round and the last pair of row tiles well, and a wave has a second superblock to
+  // load behind the first; else one row tile, by two column tiles where that leaves 192 or more
+  // workgroups. MI355X, us with the operands' launch, weights from HBM, 1 x 2 / 2 x 2 / 2 x 4:
+  //   N x K, rows         fill of 2 x 2, 2 x 4
+  //   4096 x 14336, 126   1, 1          48 / 43 / 37 (Q6_K 68 / 53 / 48)
+  //   4096 x 14336, 72    .63, .63      35 / 40 / 34
+  //   4096 x 14336, 36    .75, .38      26 / 24 / 34 (Q6_K 35 / 28 / 42)
+  //   14336 x 4096, 18    .88, .88      18 / 19 / 16
+  //   14336 x 4096, 72    .73, .73      33 / 39 / 35
+  //   14336 x 4096, 126   1, .88        49 / 49 / 46 (Q6_K 72 / 64 / 61, Q5_K 65 / 60 / 65)
+  //   2048 x 4096, 126    1, .5         11.8 / 11.1 / 14.2
+  //   5120 x 2048, 126    .83, .63      14.0 / 15.9 / 16.3 (one superblock per wave)
+  // Q5_K's 2 x 4 spills. 4 x 2 spills or leaves too few waves: 62 at the first line.
+  auto fill = [&](int ntile) {  // of the last round of CUs and of the last row pair, in 1/64
+    const int64_t pairs = (row_tiles + 1) / 2, wg = (tiles + ntile - 1) / ntile * pairs;
+    return wg * row_tiles * 64 / ((wg + 255) / 256 * 256 * pairs * 2);
+  };
+  if constexpr (NW == 8) {
+    if (S >= 2 * NW) {
+      if constexpr (FMT != FMT_Q5_K) {
+        if (fill(4) >= 56) {
+          go(kquant_gemv_mt<FMT, NW, 2, 4>, 2, 4);
+          SV_CHECK_LAUNCH();
+          return SV_OK;
+        }
+      }
+      if (fill(2) >= 48) {
+        go(kquant_gemv_mt<FMT, NW, 2, 2>, 2, 2);
+        SV_CHECK_LAUNCH();
+        return SV_OK;
+      }
+    }
+  }
+  if ((int64_t)(tiles / 2) * row_tiles >= 192) go(kquant_gemv_mt<FMT, NW, 1, 2>, 1, 2);
+  else go(kquant_gemv_mt<FMT, NW, 1, 1>, 1, 1);
   SV_CHECK_LAUNCH();
   return SV_OK;
 }

@@ -63,3 +63,25 @@ def test_q6k_every_scale_is_exact(gpu, m):
     torch.cuda.synchronize()
     want = torch.from_numpy(Q.dequant(raw, 6, n, k)).double()[:, at].T
     assert ((out.cpu().double() - want).abs() <= want.abs() * 2.0 ** -23).all()
+
+
+@pytest.mark.parametrize("fmt", [4, 5, 6, 8])
+@pytest.mark.parametrize("m,n,k", [(235, 2000, 4096), (241, 2000, 4352), (200, 2000, 4096),
+                                   (113, 2000, 4352), (33, 2000, 4352)])
+def test_wide_rows_equal_single_row_tiles(gpu, fmt, m, n, k):
+    """Blocks of two row tiles by four or two column tiles (a last pair of one tile, a last group
+    of one column tile, waves with two and three superblocks) against 16-row calls, bit for bit."""
+    from oracle import quant as Q
+    from snowllm_amd import ops
+    print(f"wide rows fmt={fmt} m={m} n={n} k={k}", flush=True)
+    make = {4: Q.make_q4_k, 5: Q.make_q5_k, 6: Q.make_q6_k, 8: Q.make_q8_0}[fmt]
+    quant, meta = ops.gemm_kquant_shuffle_b(fmt, torch.from_numpy(make(n, k, seed=m)).cuda(), n, k)
+    x = Q.make_activations(m, k, seed=k).cuda()
+    ws = torch.empty(ops.gemm_kquant_a_ws_bytes(m, k), dtype=torch.uint8, device="cuda")
+    out, want = torch.empty(m, n, device="cuda"), torch.empty(m, n, device="cuda")
+    ops.gemm_kquant_a(fmt, x, quant, meta, out, m, n, k, ws)
+    for r in range(0, m, 16):
+        c = min(16, m - r)
+        ops.gemm_kquant_a(fmt, x[r:r + c], quant, meta, want[r:r + c], c, n, k,
+                          ws[:ops.gemm_kquant_a_ws_bytes(c, k)])
+    assert torch.equal(out, want)
