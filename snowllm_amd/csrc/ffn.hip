@@ -593,6 +593,64 @@ __global__ void __launch_bounds__(WS * PPB * 64)
                                             M, F, S);
 }
 
+// The dense gate/up GEMV over more than 16 rows in one launch: blockIdx.y takes two row tiles, a
+// workgroup PG groups of P pairs (a gate and an up tile each), a group two waves that split the
+// superblocks as gate_up_kernel's do, each with both row tiles' products of every weight it
+// decodes; the waves exchange halves of their sums, so that each finishes one row tile. The same
+// products and sums, so the same bits, as gate_up_kernel per row tile. Bound: the vector units'
+// decode and rescaling and the L2 reads of the operands, as kquant_gemv_mt's; the registers hold
+// two row tiles by four column tiles at two waves per SIMD.
+constexpr int GUR_PG = 4;
+template <int FMT, int P>
+__global__ void __launch_bounds__(GUR_PG * 2 * 64) gate_up_rows_kernel(
+    const uint8_t* __restrict__ quant, const uint8_t* __restrict__ meta,
+    const void* __restrict__ ws, uint16_t* __restrict__ act_out, int M, int F, int S,
+    size_t tile_bytes) {
+  __shared__ floatx4 part[GUR_PG][2][2 * P][64];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int pl = wv >> 1, sw = wv & 1;
+  const int half_tiles = F / TILE_N;
+  const int pair0 = (blockIdx.x * GUR_PG + pl) * P;
+  const int m0 = blockIdx.y * 2;
+  const GemvStreams st = make_streams<FMT>(quant, meta, ws, 2 * half_tiles, S, lane, 16);
+  floatx4 acc[2][2 * P];
+#pragma unroll
+  for (int t = 0; t < 2 * P; ++t) acc[0][t] = acc[1][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  if (pair0 < half_tiles)
+    gemv_rows_loop<FMT, 2, 2 * P, 2>(
+        st, ws, tile_bytes, M, m0, S, lane, sw,
+        [&](int t) { return pair0 + (t >> 1) + (t & 1) * half_tiles; }, decode_magic<FMT>(), acc);
+  floatx4 own[2 * P];
+#pragma unroll
+  for (int t = 0; t < 2 * P; ++t) {
+    floatx4 other;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float a0 = acc[0][t][i], a1 = acc[1][t][i];
+      own[t][i] = sw ? a1 : a0;
+      other[i] = sw ? a0 : a1;
+    }
+    part[pl][sw][t][lane] = other;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    if (pair0 + p >= half_tiles) break;
+    const floatx4 g = own[2 * p] + part[pl][sw ^ 1][2 * p][lane];
+    const floatx4 u = own[2 * p + 1] + part[pl][sw ^ 1][2 * p + 1][lane];
+    const int n = (pair0 + p) * TILE_N + (lane & 15);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = (m0 + sw) * TILE_M + 4 * (lane >> 4) + i;
+      if (row >= M) break;
+      const float gg = bf16_to_f32(f32_to_bf16(g[i]));  // projections are bf16 tensors
+      const float uu = bf16_to_f32(f32_to_bf16(u[i]));
+      act_out[(int64_t)row * F + n] = f32_to_bf16(gg / (1.0f + __expf(-gg)) * uu);
+    }
+  }
+}
+
 // The gate/up loop by superblock count S: at S = 8 or 16 (hidden 2048 or 4096) each of a pair's
 // two waves walks its S / 2 superblocks with the weights of the next two in flight behind the
 // one it multiplies (gemv_loop_deep, unrolled), otherwise gemv_loop's one. The same sums in the
@@ -1681,6 +1739,30 @@ SV_API int snowverify_gate_up_swiglu(int fmt, const void* quant, const void* met
     else if (fmt == 6) go(gate_up_kernel<6, WS, PPB, SC>);
     else go(gate_up_kernel<8, WS, PPB, SC>);
   });
+  SV_CHECK_LAUNCH();
+  return SV_OK;
+}
+
+// The same over up to 256 rows: ws the prepared operands of ceil(M / 16) row tiles.
+SV_API int snowverify_gate_up_swiglu_rows(int fmt, const void* quant, const void* meta,
+                                          const void* ws, void* act, int64_t M, int64_t F,
+                                          int64_t K, void* stream) {
+  if (M <= 16) return snowverify_gate_up_swiglu(fmt, quant, meta, ws, act, M, F, K, stream);
+  if ((fmt != 4 && fmt != 5 && fmt != 6 && fmt != 8) || M > 256 || F <= 0 || F % 16 || K <= 0 ||
+      K % 256)
+    return SV_EINVAL;
+  const int S = (int)(K / 256);
+  auto go = [&](auto kern, int pairs) {
+    const int64_t per = GUR_PG * pairs;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((F / 16 + per - 1) / per), (unsigned)((M + 31) / 32)),
+                       dim3(GUR_PG * 2 * 64), 0, Sx(stream), (const uint8_t*)quant,
+                       (const uint8_t*)meta, ws, (uint16_t*)act, (int)M, (int)F, S,
+                       xprep_tile_bytes(S));
+  };
+  if (fmt == 4) go(gate_up_rows_kernel<4, 2>, 2);
+  else if (fmt == 5) go(gate_up_rows_kernel<5, 1>, 1);  // (two pairs spill)
+  else if (fmt == 6) go(gate_up_rows_kernel<6, 2>, 2);
+  else go(gate_up_rows_kernel<8, 2>, 2);
   SV_CHECK_LAUNCH();
   return SV_OK;
 }

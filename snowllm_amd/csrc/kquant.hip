@@ -89,8 +89,7 @@ __global__ void __launch_bounds__(NW * 64) kquant_gemv(const u32x4* __restrict__
 // ---------------------------------------------------------------------------------------
 // The same GEMV over MT 16-row tiles at once (a verify step wider than 16 rows; blockIdx.y: the
 // group of MT tiles): each wave decodes a superblock of NT column tiles once for the prepared
-// operands of MT row tiles, and the next superblock's operands load into the registers that the
-// current one's products free. Bound: the L2 reads (26 KB per 2 x 4 tiles and superblock, 13 KB
+// operands of MT row tiles (gemv_rows_loop). Bound: the L2 reads (26 KB per 2 x 4 tiles and superblock, 13 KB
 // per 1 x 2) and the vector units' decode and rescaling, both shared by more tiles the more a
 // wave holds; the registers of two waves per SIMD limit that to 2 x 4. Q4_K 4096 x 14336, 126
 // rows: 50 -> 37 us against one row tile by two column tiles with no load ahead. The per-row arithmetic and the waves' superblock split are those of
@@ -103,87 +102,18 @@ __global__ void __launch_bounds__(NW * 64) kquant_gemv_mt(const u32x4* __restric
                                                           void* __restrict__ c, int M, int N,
                                                           int S, int c_bf16, size_t tile_bytes,
                                                           int ldc) {
-  constexpr int QV = QLayout<FMT>::kQuantVecs;
   __shared__ floatx4 part[NW][NT][64];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int kq = lane >> 4, r = lane & 15;
   const int tiles = N / TILE_N;
   const int tile0 = blockIdx.x * NT;  // NT column tiles share each row tile's operands
   const int m0 = blockIdx.y * MT;
   const int row_tiles = (M + TILE_M - 1) / TILE_M;
   const GemvStreams st = make_streams<FMT>(quant, meta, ws, tiles, S, lane, 16);
-  __amdgpu_buffer_rsrc_t xr[MT], sxr[MT], scr[MT];
-  uint32_t vx[MT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    // a row tile past the last: the last one's sums and scales, and no operands
-    const int tile = m0 + m < row_tiles ? m0 + m : row_tiles - 1;
-    XPrepView xv = xprep_view((char*)ws + (size_t)tile * tile_bytes, S);
-    xr[m] = __builtin_amdgcn_make_buffer_rsrc((void*)xv.xop, 0, S * 8 * 64 * 16, 0x00020000);
-    sxr[m] = __builtin_amdgcn_make_buffer_rsrc((void*)xv.sxop, 0, S * 2 * 64 * 4, 0x00020000);
-    scr[m] = __builtin_amdgcn_make_buffer_rsrc((void*)xv.scale, 0, S * 16 * 4, 0x00020000);
-    vx[m] = r < M - (m0 + m) * TILE_M ? lane * 16 : 0x80000000u;
-  }
   const uint32_t Mv = decode_magic<FMT>();
   floatx4 acc[MT][NT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) acc[m][t] = floatx4{0.f, 0.f, 0.f, 0.f};
-  // the operands of one superblock; the next one's go into the same registers as they fall free
-  // (a tile past the last column reads nothing: its buffer offsets are out of range)
-  u32x4 q[NT][1][QV], mt4[NT][1], x[MT][8];
-  uint32_t dq[NT][1];
-  float sx0[MT], sx1[MT];
-  floatx4 sc[MT];
-  auto load_w = [&](int t, int s) {
-    load_sb_w<FMT, 1>(q[t], mt4[t], st, s, S, tile0 + t, 1);
-    if constexpr (FMT == FMT_Q6_K) load_sb_d<1>(dq[t], st, s, S, tile0 + t, 1);
-    else dq[t][0] = 0u;
-  };
-  auto load_x = [&](int m, int j, int s) {
-    x[m][j] = bload4(xr[m], vx[m], (uint32_t)((s * 8 + j) * 64 * 16));
-  };
-  auto load_sx = [&](int m, int s) {
-    sx0[m] = bload1(sxr[m], lane * 4, (uint32_t)((s * 2 + 0) * 64 * 4));
-    sx1[m] = bload1(sxr[m], lane * 4, (uint32_t)((s * 2 + 1) * 64 * 4));
-    sc[m] = __builtin_bit_cast(floatx4, bload4(scr[m], kq * 16, (uint32_t)(s * 16 * 4)));
-  };
-  auto step = [&](int s, auto more) {
-    constexpr bool MORE = decltype(more)::value;
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      floatx4 sb[MT];
-      tile_superblock_rows<FMT, MT>(
-          q[t][0], mt4[t][0], dq[t][0],
-          [&](int m, int j) {
-            const half8 v = __builtin_bit_cast(half8, x[m][j]);
-            if (MORE && t == NT - 1) load_x(m, j, s + NW);
-            return v;
-          },
-          sx0, sx1, kq, Mv, sb);
-#pragma unroll
-      for (int m = 0; m < MT; ++m) acc[m][t] += sb[m] * sc[m];
-      if (MORE) load_w(t, s + NW);
-    }
-    if (MORE)
-#pragma unroll
-      for (int m = 0; m < MT; ++m) load_sx(m, s + NW);
-  };
-  if (w < S) {
-#pragma unroll
-    for (int t = 0; t < NT; ++t) load_w(t, w);
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) load_x(m, j, w);
-      load_sx(m, w);
-    }
-    int s = w;
-    for (; s + NW < S; s += NW) step(s, std::true_type{});
-    step(s, std::false_type{});
-  }
+  gemv_rows_loop<FMT, MT, NT, NW>(st, ws, tile_bytes, M, m0, S, lane, w,
+                                  [&](int t) { return tile0 + t; }, Mv, acc);
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
     if (m0 + m >= row_tiles) break;  // uniform

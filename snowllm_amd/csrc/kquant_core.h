@@ -11,6 +11,8 @@
 // v_mfma_f32_16x16x4_f32 with the sub-block sums of the activations. Activations are
 // converted to fp16 with a power-of-two scale per (row, superblock): exact for bf16 input.
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 
 namespace kq {
@@ -606,6 +608,85 @@ __device__ __forceinline__ void gemv_loop(const GemvStreams& st, int w, int S, i
     s += NW;
     if (s >= S) break;
   }
+}
+
+// Wave w of NW walks superblocks w, w + NW, ... of NT column tiles tile_of(t) for the MT row tiles
+// from m0, of which M rows exist; row tile m's operands lie at ws + m * tile_bytes. Each weight is
+// decoded once for the MT row tiles, and the next superblock's operands load into the registers
+// that the current one's products free. acc[m][t]: this wave's sums, those of the one-tile loops.
+template <int FMT, int MT, int NT, int NW, class TileOf>
+__device__ __forceinline__ void gemv_rows_loop(const GemvStreams& st, const void* ws,
+                                               size_t tile_bytes, int M, int m0, int S, int lane,
+                                               int w, TileOf&& tile_of, uint32_t Mv,
+                                               floatx4 (&acc)[MT][NT]) {
+  const int kq = lane >> 4, r = lane & 15;
+  const int row_tiles = (M + TILE_M - 1) / TILE_M;
+  __amdgpu_buffer_rsrc_t xr[MT], sxr[MT], scr[MT];
+  uint32_t vx[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    // a row tile past the last: the last one's sums and scales, and no operands
+    const int tile = m0 + m < row_tiles ? m0 + m : row_tiles - 1;
+    XPrepView xv = xprep_view((char*)ws + (size_t)tile * tile_bytes, S);
+    xr[m] = __builtin_amdgcn_make_buffer_rsrc((void*)xv.xop, 0, S * 8 * 64 * 16, 0x00020000);
+    sxr[m] = __builtin_amdgcn_make_buffer_rsrc((void*)xv.sxop, 0, S * 2 * 64 * 4, 0x00020000);
+    scr[m] = __builtin_amdgcn_make_buffer_rsrc((void*)xv.scale, 0, S * 16 * 4, 0x00020000);
+    vx[m] = r < M - (m0 + m) * TILE_M ? lane * 16 : 0x80000000u;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[m][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+  // (a tile past the last column reads nothing: its buffer offsets are out of range)
+  u32x4 q[NT][1][QLayout<FMT>::kQuantVecs], mt4[NT][1], x[MT][8];
+  uint32_t dq[NT][1];
+  float sx0[MT], sx1[MT];
+  floatx4 sc[MT];
+  auto load_w = [&](int t, int s) {
+    load_sb_w<FMT, 1>(q[t], mt4[t], st, s, S, tile_of(t), 1);
+    if constexpr (FMT == FMT_Q6_K) load_sb_d<1>(dq[t], st, s, S, tile_of(t), 1);
+    else dq[t][0] = 0u;
+  };
+  auto load_x = [&](int m, int j, int s) {
+    x[m][j] = bload4(xr[m], vx[m], (uint32_t)((s * 8 + j) * 64 * 16));
+  };
+  auto load_sx = [&](int m, int s) {
+    sx0[m] = bload1(sxr[m], lane * 4, (uint32_t)((s * 2 + 0) * 64 * 4));
+    sx1[m] = bload1(sxr[m], lane * 4, (uint32_t)((s * 2 + 1) * 64 * 4));
+    sc[m] = __builtin_bit_cast(floatx4, bload4(scr[m], kq * 16, (uint32_t)(s * 16 * 4)));
+  };
+  auto step = [&](int s, auto more) {
+    constexpr bool MORE = decltype(more)::value;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      floatx4 sb[MT];
+      tile_superblock_rows<FMT, MT>(
+          q[t][0], mt4[t][0], dq[t][0],
+          [&](int m, int j) {
+            const half8 v = __builtin_bit_cast(half8, x[m][j]);
+            if (MORE && t == NT - 1) load_x(m, j, s + NW);
+            return v;
+          },
+          sx0, sx1, kq, Mv, sb);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) acc[m][t] += sb[m] * sc[m];
+      if (MORE) load_w(t, s + NW);
+    }
+    if (MORE)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) load_sx(m, s + NW);
+  };
+  if (w >= S) return;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) load_w(t, w);
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) load_x(m, j, w);
+    load_sx(m, w);
+  }
+  int s = w;
+#pragma unroll 1
+  for (; s + NW < S; s += NW) step(s, std::true_type{});
+  step(s, std::false_type{});
 }
 
 // Wave w of NW walks SC superblocks (w, w + NW, ...) of the tiles tile0 + t * tstride with the

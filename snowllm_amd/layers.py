@@ -125,6 +125,12 @@ def gate_up_swiglu(fmt, quant, meta, ws, act, M, F, K):
                                         _stream()), "gate_up_swiglu")
 
 
+def gate_up_swiglu_rows(fmt, quant, meta, ws, act, M, F, K):
+    _chk(act, "activation", torch.bfloat16, M, F)
+    check(lib.snowverify_gate_up_swiglu_rows(fmt, _p(quant), _p(meta), _p(ws), _p(act), M, F, K,
+                                             _stream()), "gate_up_swiglu_rows")
+
+
 def swiglu(gate_up, out):
     M, F = out.shape
     check(lib.snowverify_swiglu(_p(gate_up), gate_up.stride(0), _p(out), M, F, _stream()), "swiglu")

@@ -242,8 +242,8 @@ class VerifyModel:
         self.head_fmt = 0
         # MoE layers: post-attention norm, router and routing/plan in one launch where the
         # fused kernel takes the shape (False: the three separate launches, the same bits)
-        # the MoE and the 16-bit GEMVs take at most 16 rows per launch: a step of more rows
-        # runs them on row chunks (the fused router on chunks whose rows fit its LDS)
+        # the MoE runs on row chunks (the fused router on chunks whose rows fit its LDS); the
+        # other layers' launches take every row
         M = batch * c.block
         self.rows = M
         self.row_chunks = [(r0, min(16, M - r0)) for r0 in range(0, M, 16)]
@@ -550,10 +550,8 @@ class VerifyModel:
             else:
                 Lops.norm_prep(self.o, lw.post_norm, self.ws_h2, c.eps, res_in=res_in,
                                res_out=res_out)
-                for r0, n in self.row_chunks:
-                    Lops.gate_up_swiglu(gu_fmt, lw.gu[0], lw.gu[1],
-                                        self._ws_rows(self.ws_h2, r0), self.act[r0:r0 + n], n,
-                                        c.ffn, H)
+                Lops.gate_up_swiglu_rows(gu_fmt, lw.gu[0], lw.gu[1], self.ws_h2, self.act, T,
+                                         c.ffn, H)
                 ops.gemm_kquant_a(dn_fmt, self.act, lw.dn[0], lw.dn[1], self.x, T,
                                   H, c.ffn, self.ws_act)
             res_in, res_out = res_out, self.res[1] if res_out is self.res[0] else self.res[0]

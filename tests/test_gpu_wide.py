@@ -85,3 +85,28 @@ def test_wide_rows_equal_single_row_tiles(gpu, fmt, m, n, k):
         ops.gemm_kquant_a(fmt, x[r:r + c], quant, meta, want[r:r + c], c, n, k,
                           ws[:ops.gemm_kquant_a_ws_bytes(c, k)])
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("fmt", [4, 5, 6, 8])
+@pytest.mark.parametrize("m,f,k", [(17, 272, 4096), (33, 144, 2048), (128, 1040, 1280),
+                                   (256, 16, 256)])
+def test_gate_up_rows_equal_row_chunks(gpu, fmt, m, f, k):
+    """Gate/up over many rows in one launch (a last pair of one row tile, a last group of one
+    column pair, a wave without a superblock) against 16-row launches, bit for bit."""
+    from oracle import quant as Q
+    from snowllm_amd import layers as L, ops
+    print(f"gate_up rows fmt={fmt} m={m} f={f} k={k}", flush=True)
+    make = {4: Q.make_q4_k, 5: Q.make_q5_k, 6: Q.make_q6_k, 8: Q.make_q8_0}[fmt]
+    raw = torch.from_numpy(make(2 * f, k, seed=m)).cuda()
+    quant, meta = ops.gemm_kquant_shuffle_b(fmt, raw, 2 * f, k)
+    x = Q.make_activations(m, k, seed=k).cuda()
+    ws = torch.empty(ops.gemm_kquant_a_ws_bytes(m, k), dtype=torch.uint8, device="cuda")
+    ops.gemm_kquant_prepare_a(x, ws)
+    out = torch.empty(m, f, dtype=torch.bfloat16, device="cuda")
+    want = torch.empty_like(out)
+    L.gate_up_swiglu_rows(fmt, quant, meta, ws, out, m, f, k)
+    tile = ops.gemm_kquant_a_ws_bytes(16, k)
+    for r in range(0, m, 16):
+        c = min(16, m - r)
+        L.gate_up_swiglu(fmt, quant, meta, ws[r // 16 * tile:], want[r:r + c], c, f, k)
+    assert torch.equal(out, want)
