@@ -600,7 +600,7 @@ int snowverify_dense_gemv(int wt, const void* w, const void* act, void* c, int64
 /* act[M, F] = silu(x Wg^T) * (x Wu^T), gate_up the packed [2F, K] k-quant weight. */
 int snowverify_gate_up_swiglu(int fmt, const void* quant, const void* meta, const void* ws,
                               void* act, int64_t M, int64_t F, int64_t K, void* stream);
-/* The same for M <= 256 rows (operands of ceil(M / 16) row tiles) in one launch. */
+/* The same for M <= 256 rows (operands of ceil(M / 16) row tiles). */
 int snowverify_gate_up_swiglu_rows(int fmt, const void* quant, const void* meta, const void* ws,
                                    void* act, int64_t M, int64_t F, int64_t K, void* stream);
 /* MoE: plan of the experts the block touches (device side), then the experts of one layer.

@@ -599,7 +599,8 @@ __global__ void __launch_bounds__(WS * PPB * 64)
 // decodes; the waves exchange halves of their sums, so that each finishes one row tile. The same
 // products and sums, so the same bits, as gate_up_kernel per row tile. Bound: the vector units'
 // decode and rescaling and the L2 reads of the operands, as kquant_gemv_mt's; the registers hold
-// two row tiles by four column tiles at two waves per SIMD.
+// two row tiles by four column tiles at two waves per SIMD. F 14,336, K 4096, Q4_K, 108 rows: 66
+// us against 110 for seven 16-row launches.
 constexpr int GUR_PG = 4;
 template <int FMT, int P>
 __global__ void __launch_bounds__(GUR_PG * 2 * 64) gate_up_rows_kernel(
@@ -1752,6 +1753,22 @@ SV_API int snowverify_gate_up_swiglu_rows(int fmt, const void* quant, const void
       K % 256)
     return SV_EINVAL;
   const int S = (int)(K / 256);
+  // Few rows on few workgroups go tile by tile: one launch takes as long as two or three there.
+  // MI355X, us, 16-row launches / one launch, Q4_K: F 14,336, K 4096: 18 rows 33 / 36, 36 rows
+  // 48 / 36, 108 rows 110 / 66, 250 rows 250 / 130; F 512, K 2048: 18 rows 11 / 17, 48 rows
+  // 16.5 / 17.8, 72 rows 27 / 18; F 6144, K 2048: 36 rows 18.6 / 18.7, 72 rows 30 / 19. Q5_K
+  // (one pair per wave, so twice the workgroups): 18 rows 43 / 28, 13.9 / 12.7, 15.4 / 13.8.
+  const bool wide = M > 48 || (M > 32 && (F / 16 + 7) / 8 * 2 >= 192) || fmt == 5;
+  if (!wide) {
+    const size_t tb = xprep_tile_bytes(S);
+    for (int64_t r = 0; r < M; r += 16) {
+      const int rc = snowverify_gate_up_swiglu(fmt, quant, meta, (const char*)ws + r / 16 * tb,
+                                               (uint16_t*)act + r * F, M - r < 16 ? M - r : 16, F,
+                                               K, stream);
+      if (rc != SV_OK) return rc;
+    }
+    return SV_OK;
+  }
   auto go = [&](auto kern, int pairs) {
     const int64_t per = GUR_PG * pairs;
     hipLaunchKernelGGL(kern, dim3((unsigned)((F / 16 + per - 1) / per), (unsigned)((M + 31) / 32)),

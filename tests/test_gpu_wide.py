@@ -88,8 +88,8 @@ def test_wide_rows_equal_single_row_tiles(gpu, fmt, m, n, k):
 
 
 @pytest.mark.parametrize("fmt", [4, 5, 6, 8])
-@pytest.mark.parametrize("m,f,k", [(17, 272, 4096), (33, 144, 2048), (128, 1040, 1280),
-                                   (256, 16, 256)])
+@pytest.mark.parametrize("m,f,k", [(17, 272, 4096), (33, 144, 2048), (33, 12400, 512),
+                                   (113, 1040, 1280), (256, 16, 256)])
 def test_gate_up_rows_equal_row_chunks(gpu, fmt, m, f, k):
     """Gate/up over many rows in one launch (a last pair of one row tile, a last group of one
     column pair, a wave without a superblock) against 16-row launches, bit for bit."""
