@@ -191,8 +191,9 @@ __global__ void __launch_bounds__(NT) softmax_norm(float* __restrict__ dense, in
   }
 }
 
-// Exclusive block scan of u64 run sums for blockDim == N (buf: one slot per wave); returns the
-// exclusive prefix.
+// Exclusive block scan of u64 run sums for blockDim == N (buf: one slot per wave, in no other use
+// between the barriers before and after the call); returns the exclusive prefix. Every thread
+// calls it.
 template <int N>
 __device__ uint64_t block_exclusive_scan_u64(uint64_t v, uint64_t* buf) {
   const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
@@ -227,6 +228,7 @@ struct TopkShared {
   uint64_t sel_key[TOPK_CAP];  // (ord key << 32) | ~index : descending order == wanted order
   uint64_t sorted[TOPK_MAX];
   uint64_t red[TOPK_NT / WAVE];
+  uint64_t scan[TOPK_NT / WAVE];  // apart from red: the scan ends without a barrier
   uint32_t hist[256];
   uint32_t count[16][3];
   uint16_t active[TOPK_NT];
@@ -550,7 +552,8 @@ __global__ void __launch_bounds__(TOPK_NT) topk_topp_rows(
     // keep i iff the exclusive prefix (sorted order) is below top_p
     const double limit = (double)tp * (double)(1ull << SV_FIX_BITS);
     const uint64_t f = t < k ? canon_fix(v) : 0ull;
-    const bool kept = t < k && (double)block_exclusive_scan_u64<TOPK_NT>(f, sh.red) < limit;
+    const uint64_t pre = block_exclusive_scan_u64<TOPK_NT>(f, sh.scan);  // every thread: barriers
+    const bool kept = t < k && (double)pre < limit;
     const float Kf = canon_unfix(block_sum_u64<TOPK_NT>(kept ? f : 0ull, sh.red));
     v = (kept && Kf > 0.0f) ? canon_div(v, Kf) : 0.0f;
   }

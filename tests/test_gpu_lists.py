@@ -53,6 +53,14 @@ def test_short_lists(gpu, V, k):
     _check(V, [min(k, V)] * 7, [0.9, 1.0, 0.95, 0.8, 0.7, 0.5, 0.99], V + k)
 
 
+@pytest.mark.parametrize("V", [1030, 50257])
+@pytest.mark.parametrize("k", [65, 100, 300, 1000])
+def test_short_lists_of_several_waves_cut_by_top_p(gpu, V, k):
+    """More list slots than one wave holds (and fewer than the workgroup's threads), cut within the
+    first wave, at its end and waves later: the prefix scan and the kept sum run in every wave."""
+    _check(V, [k] * 7, [0.02, 0.3, 0.001, 0.1, 0.6, 64.0 / k, 0.9], V + k)
+
+
 @pytest.mark.parametrize("V", [1100, 8193, 32000, 151937])
 def test_wide_lists(gpu, V):
     """The whole vocabulary with top-p, widths between, short lists beside them."""
