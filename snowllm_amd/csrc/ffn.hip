@@ -225,7 +225,8 @@ __global__ void __launch_bounds__(NW * 64) dense_gemv(const u32x4* __restrict__ 
     for (int t = 0; t < NTILE; ++t)
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        wb[t][j] = bload4(wr, lane * 16, (uint32_t)(((t * S + s) * 8 + j) * 64 * 16));
+        wb[t][j] = bload4(wr, lane * 16,
+                          (uint32_t)((((t < own ? t : own - 1) * S + s) * 8 + j) * 64 * 16));
     u32x4 xa[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -331,7 +332,7 @@ dense_gemv_wide(const u32x4* __restrict__ w, const void* __restrict__ act, void*
     for (int t = 0; t < NT; ++t)
       wb[b][t] = __builtin_bit_cast(
           u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, s < S ? vw : 0x80000000u,
-                                                       s < S ? (uint32_t)(((t * S + s) * 8 + j) * 64 * 16) : 0u,
+                                                       s < S ? (uint32_t)((((t < own ? t : own - 1) * S + s) * 8 + j) * 64 * 16) : 0u,
                                                        2 /* nt */));
   };
 #pragma unroll
@@ -614,7 +615,8 @@ __global__ void __launch_bounds__(GUR_PG * 2 * 64) gate_up_rows_kernel(
   const int half_tiles = F / TILE_N;
   const int pair0 = (blockIdx.x * GUR_PG + pl) * P;
   const int m0 = blockIdx.y * 2;
-  const GemvStreams st = make_streams<FMT>(quant, meta, ws, 2 * half_tiles, S, lane, 16);
+  GemvStreams st = make_streams<FMT>(quant, meta, ws, 2 * half_tiles, S, lane, 16);
+  if constexpr (P > 1) st.last = 2 * half_tiles - 1;
   floatx4 acc[2][2 * P];
 #pragma unroll
   for (int t = 0; t < 2 * P; ++t) acc[0][t] = acc[1][t] = floatx4{0.f, 0.f, 0.f, 0.f};

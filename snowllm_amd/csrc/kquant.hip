@@ -39,8 +39,8 @@ __global__ void __launch_bounds__(64) xprep_kernel(const uint16_t* __restrict__ 
 }
 
 // NW waves split the superblocks of NTILE column tiles; the waves' partial sums meet in LDS
-// and are added in a fixed order. Reads past the end of a buffer return zero (buffer range
-// checking), so the last partial tile group needs no clamping.
+// and are added in a fixed order. A last partial tile group reads its last tile again and
+// writes it once.
 // RAW: ws is the bf16 activation matrix [M, S*256] itself, converted in-kernel (one launch
 // for the whole operator instead of a prep pass + GEMV).
 template <int FMT, int NTILE, int NW, bool RAW = false>
@@ -55,7 +55,8 @@ __global__ void __launch_bounds__(NW * 64) kquant_gemv(const u32x4* __restrict__
   const int kq = lane >> 4;
   const int tiles = N / TILE_N;
   const int tile0 = blockIdx.x * NTILE;
-  const GemvStreams st = make_streams<FMT>(quant, meta, ws, tiles, S, lane, M);
+  GemvStreams st = make_streams<FMT>(quant, meta, ws, tiles, S, lane, M);
+  if constexpr (NTILE > 1) st.last = tiles - 1;
   const uint32_t Mv = decode_magic<FMT>();
   floatx4 acc[NTILE];
 #pragma unroll
@@ -109,7 +110,8 @@ __global__ void __launch_bounds__(NW * 64) kquant_gemv_mt(const u32x4* __restric
   const int tile0 = blockIdx.x * NT;  // NT column tiles share each row tile's operands
   const int m0 = blockIdx.y * MT;
   const int row_tiles = (M + TILE_M - 1) / TILE_M;
-  const GemvStreams st = make_streams<FMT>(quant, meta, ws, tiles, S, lane, 16);
+  GemvStreams st = make_streams<FMT>(quant, meta, ws, tiles, S, lane, 16);
+  if constexpr (NT > 1) st.last = tiles - 1;
   const uint32_t Mv = decode_magic<FMT>();
   floatx4 acc[MT][NT];
   gemv_rows_loop<FMT, MT, NT, NW>(st, ws, tile_bytes, M, m0, S, lane, w,

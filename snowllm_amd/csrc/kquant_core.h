@@ -466,6 +466,7 @@ struct GemvStreams {
   __amdgpu_buffer_rsrc_t dmeta;  // Q6_K: the fp16 d per (tile-superblock, column)
   uint32_t v_quant, v_meta, v_xop, v_sx, v_scale;  // per-lane byte offsets
   uint32_t v_dq;  // Q6_K: this lane's column's d word
+  int last;       // the last column tile to load (callers whose groups may end past the weight's)
   uint32_t v_scale_g[4];  // row-gathered streams: offsets of the scales of rows 4*kq + i
 };
 
@@ -486,6 +487,12 @@ __device__ __forceinline__ void load_sb_x(SbOperands<FMT, NTILE>& o, const GemvS
   }
 }
 
+// A column tile past the last one: the last one again (its products are not written). The tile
+// sits in the loads' scalar offset, which the bounds check of a raw buffer load need not cover.
+__device__ __forceinline__ int group_tile(const GemvStreams& st, int tile) {
+  return tile < st.last ? tile : st.last;
+}
+
 // The weights of superblock s for tiles tile0 + t * tstride (t < NTILE).
 template <int FMT, int NTILE>
 __device__ __forceinline__ void load_sb_w(u32x4 (&q)[NTILE][QLayout<FMT>::kQuantVecs],
@@ -495,7 +502,7 @@ __device__ __forceinline__ void load_sb_w(u32x4 (&q)[NTILE][QLayout<FMT>::kQuant
   constexpr uint32_t TB = QLayout<FMT>::kTsBytes;
 #pragma unroll
   for (int t = 0; t < NTILE; ++t) {
-    const uint32_t ts = (uint32_t)((tile0 + t * tstride) * S + s);
+    const uint32_t ts = (uint32_t)(group_tile(st, tile0 + t * tstride) * S + s);
     if constexpr (FMT == FMT_Q5_K) {
       q[t][0] = bload4(st.quant, st.v_quant, ts * TB);
       q[t][1] = bload4(st.quant, st.v_quant, ts * TB + 1024);
@@ -515,7 +522,7 @@ __device__ __forceinline__ void load_sb_d(uint32_t (&dq)[NTILE], const GemvStrea
                                           int S, int tile0, int tstride) {
 #pragma unroll
   for (int t = 0; t < NTILE; ++t) {
-    const uint32_t ts = (uint32_t)((tile0 + t * tstride) * S + s);
+    const uint32_t ts = (uint32_t)(group_tile(st, tile0 + t * tstride) * S + s);
     dq[t] = bload1u(st.dmeta, st.v_dq, ts * 16 * 2);
   }
 }
@@ -572,6 +579,7 @@ __device__ __forceinline__ GemvStreams make_streams(const void* quant, const voi
   st.dmeta = __builtin_amdgcn_make_buffer_rsrc((char*)meta + mn, 0,
                                                (int)(uint32_t)(mn / 8 < 0xFFFFFFFFll ? mn / 8 : 0xFFFFFFFFll),
                                                0x00020000);
+  st.last = 0x7fffffff;  // (no clamp: a caller's groups lie within the weight unless it sets one)
   st.v_dq = (uint32_t)((r & ~1) * 2);
   st.v_quant = lane * 16;
   st.v_meta = r * 16;
@@ -635,7 +643,6 @@ __device__ __forceinline__ void gemv_rows_loop(const GemvStreams& st, const void
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[m][t] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
-  // (a tile past the last column reads nothing: its buffer offsets are out of range)
   u32x4 q[NT][1][QLayout<FMT>::kQuantVecs], mt4[NT][1], x[MT][8];
   uint32_t dq[NT][1];
   float sx0[MT], sx1[MT];

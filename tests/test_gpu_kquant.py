@@ -179,6 +179,38 @@ def test_q5k_q6k_config2_shape_and_forms(gpu, fmt):
         assert Q.rel_l2(c2.cpu().numpy(), want) < TOL, v
 
 
+# column groups that end past the weight: four and two tiles by eight waves, two by four; above 16
+# rows one row tile by two columns and two by two or four
+@pytest.mark.parametrize("fmt,m,n,k", [
+    (4, 9, 16 * 769, 2048), (4, 16, 16 * 385, 4096), (5, 9, 16 * 257, 2048),
+    (6, 9, 16 * 257, 2048), (8, 9, 16 * 257, 2048), (6, 9, 16 * 513, 1024), (8, 9, 16 * 513, 1024),
+    (4, 48, 16 * 257, 2048), (6, 33, 16 * 257, 1024), (6, 250, 16 * 129, 4096),
+    (8, 241, 16 * 127, 4096), (5, 241, 16 * 129, 4096)])
+def test_last_column_group_past_the_weight(gpu, fmt, m, n, k):
+    """The last group's missing tiles read the last tile again and are not written: the bits do
+    not depend on what lies behind the weight or behind the output."""
+    from snowllm_amd import ops
+    print(f"last group fmt={fmt} m={m} n={n} k={k}", flush=True)
+    raw = Q.make(fmt, n, k, seed=n)
+    packed = ops.gemm_kquant_shuffle_b(fmt, torch.from_numpy(raw).cuda(), n, k)
+    x = Q.make_activations(m, k, seed=m).cuda()
+    ws = torch.empty(ops.gemm_kquant_a_ws_bytes(m, k), dtype=torch.uint8, device="cuda")
+    outs = []
+    for fill in (0, 0xff):   # other data right behind the weight: zeros, then NaN patterns
+        behind = [torch.full((p.numel() + 65536,), fill, dtype=torch.uint8, device="cuda")
+                  for p in packed]
+        for b, p in zip(behind, packed):
+            b[:p.numel()].copy_(p.view(-1).view(torch.uint8))
+        quant, meta = (b[:p.numel()] for b, p in zip(behind, packed))
+        buf = torch.full((m * n + 4096,), -7.0, device="cuda")
+        ops.gemm_kquant_a(fmt, x, quant, meta, buf[:m * n].view(m, n), m, n, k, ws)
+        assert (buf[m * n:] == -7.0).all()
+        outs.append(buf[:m * n].view(m, n).cpu())
+    assert torch.equal(*outs)
+    want = Q.gemv_reference(x.cpu(), Q.dequant(raw, fmt, n, k))
+    assert Q.rel_l2(outs[0].numpy(), want) < TOL
+
+
 @pytest.mark.parametrize("m", [9, 40])   # one row tile; the wide-block form (three tiles)
 def test_strided_gemv_fills_columns(gpu, m):
     """snowverify_gemm_kquant_a_prepared_ld: a Q4_K q|k weight and a Q6_K v weight fill their
