@@ -407,15 +407,93 @@ __device__ __forceinline__ void tile_superblock_rows(const u32x4* qv, u32x4 meta
   }
 }
 
-// One row tile.
+// One row tile: the products and sums of tile_superblock_rows (every width gives a row the same
+// bits). Q4_K, Q5_K and Q8_0 are written out, not taken from there with MT = 1: the same
+// operations, but in an order for which the compiler schedules the MoE experts of 18 to 64 rows
+// 0.5 to 1.3 % faster (MI355X, Q4_K, us: 24 rows 70.0 -> 69.2, 45 rows 99.0 -> 98.0, 64 rows
+// 116.2 -> 115.4) and the Q4_K experts of other hidden sizes spill no register.
 template <int FMT>
 __device__ __forceinline__ floatx4 tile_superblock(const u32x4* qv, u32x4 meta, uint32_t dq,
                                                    const half8* xa, float sx0, float sx1, int kq,
                                                    uint32_t M) {
-  floatx4 out[1];
-  tile_superblock_rows<FMT, 1>(qv, meta, dq, [&](int, int j) { return xa[j]; }, &sx0, &sx1, kq, M,
-                               out);
-  return out[0];
+  if constexpr (FMT == FMT_Q6_K) {
+    floatx4 out[1];
+    tile_superblock_rows<FMT, 1>(qv, meta, dq, [&](int, int j) { return xa[j]; }, &sx0, &sx1, kq,
+                                 M, out);
+    return out[0];
+  }
+  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+  floatx4 acc = zero;
+  float a[8];
+  float beta_lo, beta_hi;  // beta for sub-blocks kq and kq + 4
+  if constexpr (FMT == FMT_Q4_K || FMT == FMT_Q5_K) {
+    const float d = f16_to_f32((uint16_t)(meta.x & 0xffff));
+    const float dmin = f16_to_f32((uint16_t)(meta.x >> 16));
+    const uint32_t s0 = meta.y, s1 = meta.z, s2 = meta.w;
+    const uint32_t sc03 = s0 & 0x3f3f3f3fu;
+    const uint32_t m03 = s1 & 0x3f3f3f3fu;
+    const uint32_t sc47 = (s2 & 0x0f0f0f0fu) | ((s0 >> 2) & 0x30303030u);
+    const uint32_t m47 = ((s2 >> 4) & 0x0f0f0f0fu) | ((s1 >> 2) & 0x30303030u);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      a[i] = d * byte_f(sc03, i);
+      a[4 + i] = d * byte_f(sc47, i);
+    }
+    const float m_lo = dmin * byte_f(m03, kq);
+    const float m_hi = dmin * byte_f(m47, kq);
+    // even sub-blocks carry the 1024 offset; odd ones read 1024 + 16 q, i.e. 64 after the 1/16
+    const float off = (kq & 1) ? 64.0f : 1024.0f;
+    beta_lo = __builtin_fmaf(off, d * byte_f(sc03, kq), m_lo);  // a[kq] without a select chain
+    beta_hi = __builtin_fmaf(off, d * byte_f(sc47, kq), m_hi);
+    const u32x4 q0 = qv[0], q1 = qv[1];
+    half8 lo, hi;
+    floatx4 c;
+    // Q5_K: OR the fifth bits into the nibble lanes (bit 4 of 1024 + q, bit 8 of 1024 + 16 q)
+    auto fifth = [&](int j, half8& l, half8& h) {
+      if constexpr (FMT == FMT_Q5_K) {
+        uint32_t e[4];
+        q5_bits(qv[2].x, qv[2].y, j, 4, e);
+        l = or_half8(l, e);
+        q5_bits(qv[2].x, qv[2].y, j + 1, 8, e);
+        h = or_half8(h, e);
+      }
+    };
+    auto group = [&](int j, uint32_t wa, uint32_t wb) {
+      q4_group(wa, wb, M, lo, hi);
+      fifth(j, lo, hi);
+      c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[j], lo, zero, 0, 0, 0);
+      acc += a[j] * c;
+      c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[j + 1], hi, zero, 0, 0, 0);
+      acc += (a[j + 1] * 0.0625f) * c;
+    };
+    group(0, q0.x, q0.y);
+    group(2, q0.z, q0.w);
+    group(4, q1.x, q1.y);
+    group(6, q1.z, q1.w);
+  } else {
+    const uint32_t dw[4] = {meta.x, meta.y, meta.z, meta.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      a[2 * i] = f16_to_f32((uint16_t)(dw[i] & 0xffff));
+      a[2 * i + 1] = f16_to_f32((uint16_t)(dw[i] >> 16));
+    }
+    // a[kq], a[4 + kq] read straight from the packed scales (no select chain on kq)
+    beta_lo = 1152.0f * f16_to_f32((uint16_t)(((kq & 1) ? (dw[kq >> 1] >> 16) : dw[kq >> 1]) & 0xffff));
+    beta_hi = 1152.0f * f16_to_f32((uint16_t)(((kq & 1) ? (dw[2 + (kq >> 1)] >> 16) : dw[2 + (kq >> 1)]) & 0xffff));
+#pragma unroll
+    for (int jp = 0; jp < 4; ++jp) {
+      const u32x4 q = qv[jp];
+      floatx4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[2 * jp], q8_sub(q.x, q.y, M), zero, 0,
+                                                          0, 0);
+      acc += a[2 * jp] * c;
+      c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[2 * jp + 1], q8_sub(q.z, q.w, M), zero, 0, 0, 0);
+      acc += a[2 * jp + 1] * c;
+    }
+  }
+  // offset/min term: acc += (-Sx) * beta over the 8 sub-blocks (k = lane >> 4 in each half)
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sx0, beta_lo, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sx1, beta_hi, acc, 0, 0, 0);
+  return acc;
 }
 
 // Repacked weight layout per 16-column tile and superblock ("tile-superblock", ts):
