@@ -160,8 +160,10 @@ __global__ void __launch_bounds__(DSP_NT) dsp_markov_kernel(DspArgs a) {
   const int B = a.b, R = a.rank, j = a.j, G = a.nwg;
   const int col = lane & 15, kq = lane >> 4, chunks = R / 8;
   const int64_t units = (a.v + DSP_UNIT - 1) / DSP_UNIT;
-  // operand chunks 4 s + kq of the unit's rows (the tile as the buffer: chunks past the rank and
-  // units past the last read zeros without touching memory) and the unit's base logits
+  // operand chunks 4 s + kq of the unit's rows (the tile as the buffer: chunks past the rank, rows
+  // past the vocabulary and units past the last are out of its range and read zeros without
+  // touching memory; the whole offset is the vector one, which the bounds check covers) and the
+  // unit's base logits
   auto load_unit = [&](int64_t u, uint4 (&q)[KS], float (&x)[4]) {
     const int64_t tile = u * DSP_UNIT / WAVE;
     const int64_t left = a.v - tile * WAVE;
@@ -173,7 +175,7 @@ __global__ void __launch_bounds__(DSP_NT) dsp_markov_kernel(DspArgs a) {
 #pragma unroll
     for (int s = 0; s < KS; ++s)
       q[s] = __builtin_bit_cast(
-          uint4, __builtin_amdgcn_raw_buffer_load_b128(wr, at, (uint32_t)(4 * s * rows_t * 16), 0));
+          uint4, __builtin_amdgcn_raw_buffer_load_b128(wr, at + (uint32_t)(4 * s * rows_t * 16), 0, 0));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int64_t n = u * DSP_UNIT + 4 * kq + i;

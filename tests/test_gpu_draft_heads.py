@@ -102,6 +102,28 @@ def test_markov_bounds_keep_the_pick(gpu, V, rank, b, kind):
     assert np.array_equal(path.cpu().numpy(), want)
 
 
+# ranks that end inside a 32-value step of every kernel form, vocabularies that end inside a 16-row
+# unit (17 and 1 rows of the last 64-row tile)
+@pytest.mark.parametrize("V,rank", [(1041, 8), (1041, 40), (1025, 72), (1041, 136), (1025, 264)])
+def test_markov_does_not_read_past_the_weight(gpu, V, rank):
+    """Chunks past the rank and rows past the vocabulary are zeros: NaN right behind the packed
+    weight changes neither the picks nor which rows the bounds leave."""
+    from snowllm_amd.draft_heads import MarkovHead
+    _say(f"dspark markov end V={V} rank={rank}")
+    b, block = 3, 4
+    W1, W2, base, anchor, *_ = _markov_case(V, rank, b, block, V + rank)
+    head = MarkovHead(W1.cuda(), W2.cuda())
+    size = head.w2.numel() * head.w2.element_size()
+    behind = torch.full((size + 65536,), 0xff, dtype=torch.uint8, device="cuda")
+    behind[:size].copy_(head.w2.view(-1).view(torch.uint8))
+    head.w2 = behind[:size].view(head.w2.dtype).view(head.w2.shape)
+    path = torch.full((b, block), -7, dtype=torch.int64, device="cuda")
+    head.propose(None, base.cuda(), anchor.cuda(), path)
+    want = D.markov(base.numpy(), _bits(W1), _bits(W2), anchor.numpy(), block)
+    want = want[0] if isinstance(want, tuple) else want
+    assert np.array_equal(path.cpu().numpy(), want)
+
+
 def test_markov_without_confidence_and_graph_replay(gpu):
     """No confidence output; the arrival counter carries across captured replays."""
     from snowllm_amd.draft_heads import MarkovHead
