@@ -90,14 +90,18 @@ __global__ void __launch_bounds__(NW * 64) kquant_gemv(const u32x4* __restrict__
 // ---------------------------------------------------------------------------------------
 // The same GEMV over MT 16-row tiles at once (a verify step wider than 16 rows; blockIdx.y: the
 // group of MT tiles): each wave decodes a superblock of NT column tiles once for the prepared
-// operands of MT row tiles (gemv_rows_loop). Bound: the L2 reads (26 KB per 2 x 4 tiles and superblock, 13 KB
-// per 1 x 2) and the vector units' decode and rescaling, both shared by more tiles the more a
-// wave holds; the registers of two waves per SIMD limit that to 2 x 4. Q4_K 4096 x 14336, 126
-// rows: 50 -> 37 us against one row tile by two column tiles with no load ahead. The per-row arithmetic and the waves' superblock split are those of
-// kquant_gemv with NW waves, so every row gets the bits of the 16-row launch.
+// operands of MT row tiles (gemv_rows_loop). Bound: the L2 reads (26 KB per 2 x 4 tiles and
+// superblock, 13 KB per 1 x 2) and the vector units' decode and rescaling, both shared by more
+// tiles the more a wave holds. Two row tiles take the registers of two waves per SIMD, one
+// workgroup to a CU; one row tile is held to four waves per SIMD, two workgroups (above 128
+// registers Q8_0 took 10 to 15 % longer, 17.8 us against 15.3 at 5120 x 2048 and 128 rows). Q4_K
+// 4096 x 14336, 126 rows: 47 -> 38 us against one row tile by two column tiles with no load ahead.
+// The per-row arithmetic and the waves' superblock split are those of kquant_gemv with NW waves, so
+// every row gets the bits of the 16-row launch.
 // ---------------------------------------------------------------------------------------
 template <int FMT, int NW, int MT, int NT>
-__global__ void __launch_bounds__(NW * 64) kquant_gemv_mt(const u32x4* __restrict__ quant,
+__global__ void __launch_bounds__(NW * 64)
+    __attribute__((amdgpu_waves_per_eu(MT == 1 ? 4 : 2))) kquant_gemv_mt(const u32x4* __restrict__ quant,
                                                           const u32x4* __restrict__ meta,
                                                           const void* __restrict__ ws,
                                                           void* __restrict__ c, int M, int N,
@@ -114,8 +118,10 @@ __global__ void __launch_bounds__(NW * 64) kquant_gemv_mt(const u32x4* __restric
   if constexpr (NT > 1) st.last = tiles - 1;
   const uint32_t Mv = decode_magic<FMT>();
   floatx4 acc[MT][NT];
-  gemv_rows_loop<FMT, MT, NT, NW>(st, ws, tile_bytes, M, m0, S, lane, w,
-                                  [&](int t) { return tile0 + t; }, Mv, acc);
+  // (one row tile of Q8_0 has no registers for the next superblock at four waves per SIMD)
+  constexpr bool AHEAD = !(FMT == FMT_Q8_0 && MT == 1);
+  gemv_rows_loop<FMT, MT, NT, NW, AHEAD>(st, ws, tile_bytes, M, m0, S, lane, w,
+                                         [&](int t) { return tile0 + t; }, Mv, acc);
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
     if (m0 + m >= row_tiles) break;  // uniform
@@ -152,41 +158,51 @@ int launch_gemv_mt(const void* quant, const void* meta, const void* ws, void* c,
                        dim3(NW * 64), 0, s, (const u32x4*)quant, (const u32x4*)meta, ws, c, M,
                        N, S, c_bf16, tb, ldc);
   };
-  // Two row tiles by four (or two) column tiles where such workgroups, one to a CU, fill the 256
-  // CUs' last round and the last pair of row tiles well, and a wave has a second superblock to
-  // load behind the first; else one row tile, by two column tiles where that leaves 192 or more
-  // workgroups. MI355X, us with the operands' launch, weights from HBM, 1 x 2 / 2 x 2 / 2 x 4:
-  //   N x K, rows         fill of 2 x 2, 2 x 4
-  //   4096 x 14336, 126   1, 1          48 / 43 / 37 (Q6_K 68 / 53 / 48)
-  //   4096 x 14336, 72    .63, .63      35 / 40 / 34
-  //   4096 x 14336, 36    .75, .38      26 / 24 / 34 (Q6_K 35 / 28 / 42)
-  //   14336 x 4096, 18    .88, .88      18 / 19 / 16
-  //   14336 x 4096, 72    .73, .73      33 / 39 / 35
-  //   14336 x 4096, 126   1, .88        49 / 49 / 46 (Q6_K 72 / 64 / 61, Q5_K 65 / 60 / 65)
-  //   2048 x 4096, 126    1, .5         11.8 / 11.1 / 14.2
-  //   5120 x 2048, 126    .83, .63      14.0 / 15.9 / 16.3 (one superblock per wave)
-  // Q5_K's 2 x 4 spills. 4 x 2 spills or leaves too few waves: 62 at the first line.
-  auto fill = [&](int ntile) {  // of the last round of CUs and of the last row pair, in 1/64
-    const int64_t pairs = (row_tiles + 1) / 2, wg = (tiles + ntile - 1) / ntile * pairs;
-    return wg * row_tiles * 64 / ((wg + 255) / 256 * 256 * pairs * 2);
-  };
+  // One row tile per workgroup, by two column tiles where that leaves 192 or more workgroups (two
+  // of them to a CU), or two row tiles by four or two column tiles (one workgroup to a CU): the form
+  // of the least estimated time. In units of 1024 tile products, one round of the 256 CUs for
+  // 1 x 2 and 2 x 2 and half a round for 2 x 4, the estimate is the form's rounds over its speed
+  // against 1 x 2 when full. Two-row workgroups run in whole rounds; the smaller ones' last round
+  // is partly hidden. An odd last row tile costs a two-row form a whole one. The speeds and the
+  // rule are fitted to 450 sizes a format (18 N x K from 512 x 2048 to 151,936 x 2048, 17 to 256
+  // rows; MI355X, operands' launch included, weights from HBM): on average 1.0 to 1.4 % above each
+  // size's best form. Against one row tile without a load ahead 7 % (Q4_K), 4 % (Q5_K), 29 % (Q6_K)
+  // and 14 % (Q8_0) faster on average and slower nowhere, but for up to 0.4 us of 11 at 4 sizes of
+  // Q8_0; a rule on the last round's fill alone lost to it by up to 15 %. us, 1 x 2 / 2 x 2 / 2 x 4:
+  //   4096 x 14336, 126 rows   Q4_K 46 / 43 / 38      Q6_K 63 / 51 / 47
+  //   14336 x 4096, 108 rows   Q4_K 43 / 48 / 45      Q5_K 56 / 59 / -
+  //   8192 x 8192, 256 rows    Q5_K 133 / 114 / -
+  //   28672 x 4096, 240 rows   Q8_0 257 / 216 / 181
+  //   5120 x 2048, 128 rows    Q8_0 15.3 / 18.5 / 17.4
+  //   151936 x 2048, 45 rows   Q6_K 144 / 175 / 155   Q4_K 121 / 147 / 126   Q8_0 199 / 210 / 172
+  // Below eight superblocks two-row forms would leave half their waves idle. Q5_K's 2 x 4 spills
+  // and its 2 x 2 needs two superblocks per wave (K = 2048 at 240 rows: 1.16 times as long); Q4_K's
+  // and Q8_0's 2 x 2 is behind 1 x 2 or 2 x 4 everywhere.
+  const bool two = (int64_t)(tiles / 2) * row_tiles >= 192;
   if constexpr (NW == 8) {
-    if (S >= 2 * NW) {
-      if constexpr (FMT != FMT_Q5_K) {
-        if (fill(4) >= 56) {
-          go(kquant_gemv_mt<FMT, NW, 2, 4>, 2, 4);
-          SV_CHECK_LAUNCH();
-          return SV_OK;
-        }
+    const double w24 = FMT == FMT_Q4_K ? 1.1 : 1.3, w22 = FMT == FMT_Q5_K ? 1.02 : 1.1;
+    const int64_t pairs = (row_tiles + 1) / 2;
+    auto rounds = [&](int ntile) { return (double)(((tiles + ntile - 1) / ntile * pairs + 255) / 256); };
+    const int64_t small = two ? (tiles + 1) / 2 * (int64_t)row_tiles : (int64_t)tiles * row_tiles;
+    const double x = (double)small / 512, t1 = (x + (double)((small + 511) / 512)) / (two ? 2 : 4);
+    const double t24 = 2 * rounds(4) / w24, t22 = rounds(2) / w22;
+    if constexpr (FMT != FMT_Q5_K) {
+      if (t24 < t1 && (FMT != FMT_Q6_K || t24 <= t22)) {
+        go(kquant_gemv_mt<FMT, NW, 2, 4>, 2, 4);
+        SV_CHECK_LAUNCH();
+        return SV_OK;
       }
-      if (fill(2) >= 48) {
+    }
+    if constexpr (FMT == FMT_Q5_K || FMT == FMT_Q6_K) {
+      const bool deep = FMT == FMT_Q6_K || (S >= 2 * NW && rounds(2) >= 2);
+      if (deep && t22 < t1) {
         go(kquant_gemv_mt<FMT, NW, 2, 2>, 2, 2);
         SV_CHECK_LAUNCH();
         return SV_OK;
       }
     }
   }
-  if ((int64_t)(tiles / 2) * row_tiles >= 192) go(kquant_gemv_mt<FMT, NW, 1, 2>, 1, 2);
+  if (two) go(kquant_gemv_mt<FMT, NW, 1, 2>, 1, 2);
   else go(kquant_gemv_mt<FMT, NW, 1, 1>, 1, 1);
   SV_CHECK_LAUNCH();
   return SV_OK;

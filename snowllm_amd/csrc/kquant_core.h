@@ -698,9 +698,9 @@ __device__ __forceinline__ void gemv_loop(const GemvStreams& st, int w, int S, i
 
 // Wave w of NW walks superblocks w, w + NW, ... of NT column tiles tile_of(t) for the MT row tiles
 // from m0, of which M rows exist; row tile m's operands lie at ws + m * tile_bytes. Each weight is
-// decoded once for the MT row tiles, and the next superblock's operands load into the registers
+// decoded once for the MT row tiles. AHEAD: the next superblock's operands load into the registers
 // that the current one's products free. acc[m][t]: this wave's sums, those of the one-tile loops.
-template <int FMT, int MT, int NT, int NW, class TileOf>
+template <int FMT, int MT, int NT, int NW, bool AHEAD = true, class TileOf>
 __device__ __forceinline__ void gemv_rows_loop(const GemvStreams& st, const void* ws,
                                                size_t tile_bytes, int M, int m0, int S, int lane,
                                                int w, TileOf&& tile_of, uint32_t Mv,
@@ -759,15 +759,27 @@ __device__ __forceinline__ void gemv_rows_loop(const GemvStreams& st, const void
 #pragma unroll
       for (int m = 0; m < MT; ++m) load_sx(m, s + NW);
   };
+  auto load = [&](int s) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) load_w(t, s);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) load_x(m, j, s);
+      load_sx(m, s);
+    }
+  };
   if (w >= S) return;
-#pragma unroll
-  for (int t = 0; t < NT; ++t) load_w(t, w);
-#pragma unroll
-  for (int m = 0; m < MT; ++m) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) load_x(m, j, w);
-    load_sx(m, w);
+  if constexpr (!AHEAD) {
+#pragma unroll 1
+    for (int s = w; s < S; s += NW) {
+      load(s);
+      __builtin_amdgcn_sched_barrier(0);  // every load before the first product
+      step(s, std::false_type{});
+    }
+    return;
   }
+  load(w);
   int s = w;
 #pragma unroll 1
   for (; s + NW < S; s += NW) step(s, std::true_type{});

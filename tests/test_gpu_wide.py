@@ -67,10 +67,12 @@ def test_q6k_every_scale_is_exact(gpu, m):
 
 @pytest.mark.parametrize("fmt", [4, 5, 6, 8])
 @pytest.mark.parametrize("m,n,k", [(235, 2000, 4096), (241, 2000, 4352), (200, 2000, 4096),
-                                   (113, 2000, 4352), (33, 2000, 4352)])
+                                   (113, 2000, 4352), (33, 2000, 4352), (250, 2000, 2048),
+                                   (113, 2000, 2048), (200, 6160, 1280), (33, 512, 512)])
 def test_wide_rows_equal_single_row_tiles(gpu, fmt, m, n, k):
     """Blocks of two row tiles by four or two column tiles (a last pair of one tile, a last group
-    of one column tile, waves with two and three superblocks) against 16-row calls, bit for bit."""
+    of one column tile, waves with one, two and three superblocks), and blocks of one row tile (eight
+    and four waves) against 16-row calls, bit for bit."""
     from oracle import quant as Q
     from snowllm_amd import ops
     print(f"wide rows fmt={fmt} m={m} n={n} k={k}", flush=True)
