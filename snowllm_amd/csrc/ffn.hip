@@ -285,7 +285,7 @@ template <int WT, int NT, int NW, int MT>
 __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 dense_gemv_wide(const u32x4* __restrict__ w, const void* __restrict__ act, void* __restrict__ c,
                 int M, int N, int S, int c_bf16, size_t tile_bytes, int groups) {
-  constexpr int DX = 2, DW = MT == 8 && WT == WT_F16 ? 2 : 4;  // (four would spill there)
+  constexpr int DX = 2, DW = MT == 8 && WT == WT_F16 ? 2 : 4;  // (there two spill six registers already)
   __shared__ floatx4 part[NW][NT][64];
   __shared__ __attribute__((aligned(16))) float s_scale[NW][DENSE_MT * TILE_M];
   const int lane = threadIdx.x & 63;
@@ -599,9 +599,9 @@ __global__ void __launch_bounds__(WS * PPB * 64)
 // superblocks as gate_up_kernel's do, each with both row tiles' products of every weight it
 // decodes; the waves exchange halves of their sums, so that each finishes one row tile. The same
 // products and sums, so the same bits, as gate_up_kernel per row tile. Bound: the vector units'
-// decode and rescaling and the L2 reads of the operands, as kquant_gemv_mt's; the registers hold
-// two row tiles by four column tiles at two waves per SIMD. F 14,336, K 4096, Q4_K, 108 rows: 66
-// us against 110 for seven 16-row launches.
+// decode and rescaling and the L2 reads of the operands, as kquant_gemv_mt's; two row tiles by
+// four column tiles are what the registers of two waves per SIMD hold (but for eleven of Q4_K, which
+// spill). F 14,336, K 4096, Q4_K, 108 rows: 66 us against 110 for seven 16-row launches.
 constexpr int GUR_PG = 4;
 template <int FMT, int P>
 __global__ void __launch_bounds__(GUR_PG * 2 * 64) gate_up_rows_kernel(
@@ -1755,12 +1755,21 @@ SV_API int snowverify_gate_up_swiglu_rows(int fmt, const void* quant, const void
       K % 256)
     return SV_EINVAL;
   const int S = (int)(K / 256);
-  // Few rows on few workgroups go tile by tile: one launch takes as long as two or three there.
-  // MI355X, us, 16-row launches / one launch, Q4_K: F 14,336, K 4096: 18 rows 33 / 36, 36 rows
-  // 48 / 36, 108 rows 110 / 66, 250 rows 250 / 130; F 512, K 2048: 18 rows 11 / 17, 48 rows
-  // 16.5 / 17.8, 72 rows 27 / 18; F 6144, K 2048: 36 rows 18.6 / 18.7, 72 rows 30 / 19. Q5_K
-  // (one pair per wave, so twice the workgroups): 18 rows 43 / 28, 13.9 / 12.7, 15.4 / 13.8.
-  const bool wide = M > 48 || (M > 32 && (F / 16 + 7) / 8 * 2 >= 192) || fmt == 5;
+  // Two or three row tiles go tile by tile where that takes no longer. The 16-row kernel is at its
+  // best at eight superblocks (unrolled, three weight buffers), next at sixteen, and loads one
+  // superblock ahead elsewhere; one launch has few workgroups there (`groups`), of which Q5_K, one
+  // pair per wave, has twice as many. MI355X, us, weights from HBM, 16-row launches / one launch:
+  //   F 512, K 2048       Q4_K 18 rows 11 / 17, 48 rows 16.5 / 17.8, 72 rows 27 / 18; Q5_K 18 rows
+  //                       13.9 / 12.7
+  //   F 6144, K 2048      36 rows Q4_K 18.6 / 18.7, Q6_K 23.1 / 22.6, Q8_0 23.0 / 21.5
+  //   F 14,336, K 4096    18 rows Q4_K 33 / 36, Q5_K 43 / 28, Q6_K 48.6 / 45.3, Q8_0 48.4 / 45.2;
+  //                       36 rows Q4_K 48 / 36; 108 rows Q4_K 110 / 66
+  //   F 11,008, K 4096    36 rows Q4_K 47 / 38, Q6_K 66 / 44, Q8_0 65 / 42
+  //   F 28,672, K 8192    18 rows Q4_K 124 / 81, Q6_K 176 / 93, Q8_0 194 / 99
+  const int64_t groups = (F / 16 + 7) / 8 * ((M + 31) / 32);
+  const bool wide = fmt == 5 || M > 48 ||
+                    (M > 32 ? S != 8 || groups >= (fmt == 8 ? 96 : 192)
+                            : groups >= 96 && (S > 16 || (S == 16 && fmt != 4)));
   if (!wide) {
     const size_t tb = xprep_tile_bytes(S);
     for (int64_t r = 0; r < M; r += 16) {

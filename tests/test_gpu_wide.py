@@ -90,17 +90,22 @@ def test_wide_rows_equal_single_row_tiles(gpu, fmt, m, n, k):
 
 
 @pytest.mark.parametrize("fmt", [4, 5, 6, 8])
-@pytest.mark.parametrize("m,f,k", [(17, 272, 4096), (33, 144, 2048), (33, 12400, 512),
-                                   (113, 1040, 1280), (256, 16, 256)])
+# one launch at the depths that the 16-row kernel has unrolled forms for (8 and 16 superblocks: odd
+# pair counts, a last row tile of one row) and around them; the sizes where the rule changes sides
+@pytest.mark.parametrize("m,f,k", [(57, 272, 4096), (113, 144, 2048), (113, 1040, 1280),
+                                   (256, 16, 256), (33, 176, 512), (17, 272, 4096),
+                                   (33, 144, 2048), (33, 12400, 512), (20, 12288, 4096),
+                                   (45, 6144, 2048)])
 def test_gate_up_rows_equal_row_chunks(gpu, fmt, m, f, k):
     """Gate/up over many rows in one launch (a last pair of one row tile, a last group of one
-    column pair, a wave without a superblock) against 16-row launches, bit for bit."""
+    column pair, a wave without a superblock) against 16-row launches, bit for bit, and against the
+    fp64 products with the projections rounded to bf16."""
     from oracle import quant as Q
     from snowllm_amd import layers as L, ops
     print(f"gate_up rows fmt={fmt} m={m} f={f} k={k}", flush=True)
     make = {4: Q.make_q4_k, 5: Q.make_q5_k, 6: Q.make_q6_k, 8: Q.make_q8_0}[fmt]
-    raw = torch.from_numpy(make(2 * f, k, seed=m)).cuda()
-    quant, meta = ops.gemm_kquant_shuffle_b(fmt, raw, 2 * f, k)
+    host = make(2 * f, k, seed=m)
+    quant, meta = ops.gemm_kquant_shuffle_b(fmt, torch.from_numpy(host).cuda(), 2 * f, k)
     x = Q.make_activations(m, k, seed=k).cuda()
     ws = torch.empty(ops.gemm_kquant_a_ws_bytes(m, k), dtype=torch.uint8, device="cuda")
     ops.gemm_kquant_prepare_a(x, ws)
@@ -112,3 +117,10 @@ def test_gate_up_rows_equal_row_chunks(gpu, fmt, m, f, k):
         c = min(16, m - r)
         L.gate_up_swiglu(fmt, quant, meta, ws[r // 16 * tile:], want[r:r + c], c, f, k)
     assert torch.equal(out, want)
+    if f <= 1040:
+        w = torch.from_numpy(Q.dequant(host, fmt, 2 * f, k)).double()
+        y = (x.cpu().double() @ w.T).bfloat16().double()
+        exact = y[:, :f] * torch.sigmoid(y[:, :f]) * y[:, f:]
+        # the result's rounding to bf16 is 2^-9 at most; a projection that rounds the other way
+        # shifts its element by 2^-8, rarely
+        assert rel(out.cpu(), exact) < 2.0 ** -8
