@@ -24,9 +24,11 @@
 // two arrivals). Sharing the lower bound between workgroups was slower for up to eight requests
 // (its round trip costs what it saves). MI355X, us per block row with confidences, every sum in
 // fp64 before -> now: V = 151,936, rank 256: 29 -> 21 for one request, 45 -> 25 for four, 108 ->
-// 33 for eight, 188 -> 49 for sixteen; rank 64: 15.5 -> 15.1, 26 -> 18, 57 -> 23 for one, four,
-// eight; V = 32,000, rank 256: 19 -> 14, 33 -> 17, 61 -> 23. Masked logits (-inf, or the type's
-// lowest value) 45 -> 24 at four requests. Equal scores everywhere take the exact sums alone.
+// 31 for eight, 187 -> 46 for sixteen; rank 64: 14.8 -> 14.5, 26 -> 17.5, 57 -> 21 for one, four,
+// eight; V = 32,000, rank 256: 19 -> 15, 33 -> 17, 61 -> 23. Masked logits (-inf, or the type's
+// lowest value) 45 -> 24 at four requests. Equal scores everywhere (a W2 of zeros under constant
+// logits) need every row's exact sum behind the bounds: 29 -> 33, 45 -> 58 and 184 -> 116 for one,
+// four and sixteen requests, where a wave per row took 95, 290 and 1090.
 #include "common.h"
 
 namespace {
@@ -139,10 +141,69 @@ __device__ __forceinline__ uint64_t dsp_exact_key(const DspArgs& a, const float*
   return argmax_key(x + bias, (uint32_t)row);
 }
 
+// The same scores by one lane, of one row for NR requests r0, r0 + 1, ... (those from B on come out
+// as r0's), for many candidates: rows may differ from lane to lane, and neighbouring rows are
+// neighbouring words of the packed tile. The next chunks load behind the sums.
+template <int NR>
+__device__ __forceinline__ void dsp_lane_keys(const DspArgs& a, const float* s_lat, int r0,
+                                              int64_t row, uint64_t (&key)[NR]) {
+  const int chunks = a.rank / 8;
+  const int64_t tile = row / WAVE;
+  const int64_t rows_t = a.v - tile * WAVE < WAVE ? a.v - tile * WAVE : WAVE;
+  const uint4* src = (const uint4*)(a.w2 + tile * WAVE * (int64_t)a.rank) + row % WAVE;
+  const float* L[NR];
+  float x[NR];
+  double acc[NR];
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    const int r = r0 + i < a.b ? r0 + i : r0;
+    L[i] = s_lat + r * a.rank;
+    x[i] = a.base[((int64_t)r * a.block + a.j) * a.base_stride + row];
+    acc[i] = 0.0;
+  }
+  constexpr int UN = 4;  // chunks of a load
+  uint4 q[2][UN];
+  auto load = [&](int b, int cb) {
+#pragma unroll
+    for (int u = 0; u < UN; ++u) q[b][u] = src[(cb + u < chunks ? cb + u : chunks - 1) * rows_t];
+  };
+  auto sum = [&](int b, int cb) {
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      if (cb + u >= chunks) break;  // uniform
+      const uint32_t qw[4] = {q[b][u].x, q[b][u].y, q[b][u].z, q[b][u].w};
+#pragma unroll
+      for (int i = 0; i < NR; ++i) {
+        double s0 = 0.0, s1 = 0.0;  // two chains; the sum stays exact
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float* l = L[i] + (cb + u) * 8 + 2 * e;
+          s0 += (double)(__uint_as_float(qw[e] << 16) * l[0]);
+          s1 += (double)(__uint_as_float(qw[e] & 0xffff0000u) * l[1]);
+        }
+        acc[i] += s0 + s1;
+      }
+    }
+  };
+  load(0, 0);
+  for (int cb = 0; cb < chunks; cb += 2 * UN) {
+    load(1, cb + UN);
+    sum(0, cb);
+    load(0, cb + 2 * UN);
+    sum(1, cb + UN);
+  }
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    const float bias = a.fp32_bias ? (float)acc[i] : bf16_from_f64(acc[i]);
+    key[i] = argmax_key(x[i] + bias, (uint32_t)row);
+  }
+}
+
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 constexpr int DSP_UNIT = 16;              // vocabulary rows of a matrix product
 constexpr int DSP_CAND = 512;             // candidates a workgroup keeps
+constexpr int DSP_FEW = 32;               // candidates up to here are looked at in turn
 constexpr uint32_t DSP_BOTTOM = 0x007fffffu;  // ord_key(-inf)
 
 // KS: 32-value steps of the rank (values past the rank are zero operands).
@@ -154,7 +215,8 @@ __global__ void __launch_bounds__(DSP_NT) dsp_markov_kernel(DspArgs a) {
   __shared__ uint32_t s_up[DSP_CAND];            // candidates: upper bound (key), row, request
   __shared__ uint32_t s_row[DSP_CAND];
   __shared__ uint8_t s_req[DSP_CAND];
-  __shared__ uint32_t s_n, s_flag;
+  __shared__ uint16_t s_left[DSP_CAND];          // candidates that every wave's bounds leave
+  __shared__ uint32_t s_n, s_m, s_flag;
   const int t = threadIdx.x, lane = t & (WAVE - 1);
   const int w = __builtin_amdgcn_readfirstlane(t / WAVE);
   const int B = a.b, R = a.rank, j = a.j, G = a.nwg;
@@ -211,7 +273,7 @@ __global__ void __launch_bounds__(DSP_NT) dsp_markov_kernel(DspArgs a) {
     s_low[t] = 0u;
     s_best[t] = argmax_key(-__builtin_huge_valf(), (uint32_t)(blockIdx.x * DSP_WAVES * DSP_UNIT));
   }
-  if (t == 0) s_n = 0u;
+  if (t == 0) s_n = s_m = 0u;
   for (int i = t; i < B * R; i += DSP_NT) {
     const int r = i / R, e = i % R;
     const int64_t prev = j == 0 ? a.anchor[r] : a.out[(int64_t)r * a.block + j - 1];
@@ -305,10 +367,12 @@ __global__ void __launch_bounds__(DSP_NT) dsp_markov_kernel(DspArgs a) {
     o = (uint32_t)__shfl_xor((int)best, 32, WAVE);
     best = o > best ? o : best;
     low = best > low ? best : low;
+    bool full = false;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if (up[i] >= low && up[i] > DSP_BOTTOM) {
         const uint32_t at = atomicAdd(&s_n, 1u);
+        full |= at >= DSP_CAND;
         if (at < DSP_CAND) {
           s_up[at] = up[i];
           s_row[at] = (uint32_t)(u * DSP_UNIT + 4 * kq + i);
@@ -316,6 +380,7 @@ __global__ void __launch_bounds__(DSP_NT) dsp_markov_kernel(DspArgs a) {
         }
       }
     }
+    if (__ballot(full)) break;  // the exact sums of every row follow
 #pragma unroll
     for (int s = 0; s < KS; ++s) q0[s] = q1[s];
 #pragma unroll
@@ -324,24 +389,49 @@ __global__ void __launch_bounds__(DSP_NT) dsp_markov_kernel(DspArgs a) {
   if (lane < B) atomicMax(&s_low[lane], low);
   if (known) atomicMax((unsigned long long*)&s_best[col], (unsigned long long)known);
   __syncthreads();
-  // the exact scores, a wave per candidate
-  if (s_n <= DSP_CAND) {  // uniform
-    for (int i = w; i < (int)s_n; i += DSP_WAVES) {
-      const int r = s_req[i];
-      if (s_up[i] < s_low[r]) continue;
-      const uint64_t key = dsp_exact_key(a, s_lat + r * R, r, s_row[i]);
-      if (lane == 0) atomicMax((unsigned long long*)&s_best[r], (unsigned long long)key);
+  // the exact scores of the candidates that the workgroup's lower bounds leave
+  auto best_of = [&](int r, uint64_t key) {
+    if (key > s_best[r]) atomicMax((unsigned long long*)&s_best[r], (unsigned long long)key);
+  };
+  auto by_wave = [&](int c) {  // one candidate by a wave: one round trip to memory
+    const int r = s_req[c];
+    const uint64_t key = dsp_exact_key(a, s_lat + r * R, r, s_row[c]);
+    if (lane == 0) best_of(r, key);
+  };
+  const int n = (int)s_n;  // (uniform, as every branch on it)
+  if (n <= DSP_FEW) {
+    for (int c = w; c < n; c += DSP_WAVES)
+      if (s_up[c] >= s_low[s_req[c]]) by_wave(c);
+  } else if (n <= DSP_CAND) {
+    for (int c = t; c < n; c += DSP_NT)
+      if (s_up[c] >= s_low[s_req[c]]) s_left[atomicAdd(&s_m, 1u)] = (uint16_t)c;
+    __syncthreads();
+    const int m = (int)s_m;
+    if (m <= DSP_FEW / 2) {
+      for (int i = w; i < m; i += DSP_WAVES) by_wave(s_left[i]);
+    } else {  // near ties (equal scores): a lane each
+      for (int i = w * WAVE; i < m; i += DSP_NT) {
+        const int c = s_left[i + lane < m ? i + lane : m - 1], r = s_req[c];
+        uint64_t key[1];
+        dsp_lane_keys<1>(a, s_lat, r, s_row[c], key);
+        best_of(r, key[0]);
+      }
     }
   } else {
-    // too many near the top (equal scores): every row of this workgroup
-    for (int64_t v0 = (int64_t)blockIdx.x * DSP_WAVES; v0 < units; v0 += (int64_t)G * DSP_WAVES)
-      for (int i = w; i < DSP_WAVES * DSP_UNIT * B; i += DSP_WAVES) {
-        const int r = i / (DSP_WAVES * DSP_UNIT);
-        const int64_t row = v0 * DSP_UNIT + i % (DSP_WAVES * DSP_UNIT);
-        if (row >= a.v) continue;
-        const uint64_t key = dsp_exact_key(a, s_lat + r * R, r, row);
-        if (lane == 0) atomicMax((unsigned long long*)&s_best[r], (unsigned long long)key);
-      }
+    // more than the workgroup keeps (equal scores, several requests): every row, a lane each
+    const int64_t tiles = (a.v + WAVE - 1) / WAVE;
+    const int own = (int)((tiles - blockIdx.x + G - 1) / G);
+    constexpr int NR = 4;
+    const int parts = (B + NR - 1) / NR;
+    for (int p = w; p < own * parts; p += DSP_WAVES) {
+      const int r0 = p % parts * NR;
+      const int64_t row = (blockIdx.x + (int64_t)(p / parts) * G) * WAVE + lane;
+      uint64_t key[NR];
+      dsp_lane_keys<NR>(a, s_lat, r0, row < a.v ? row : a.v - 1, key);
+#pragma unroll
+      for (int i = 0; i < NR; ++i)
+        if (r0 + i < B) best_of(r0 + i, key[i]);
+    }
   }
   __syncthreads();
   uint64_t* wg_keys = a.partial;                          // [b][G]

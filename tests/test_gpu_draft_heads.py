@@ -69,11 +69,11 @@ def test_markov_equals_oracle(gpu, V, rank, b, block, pad, fp32):
 
 
 @pytest.mark.parametrize("kind", ["plain", "-inf", "lowest", "equal", "zeros", "infinite", "tiny"])
-@pytest.mark.parametrize("V,rank,b", [(77, 8, 16), (9000, 72, 5), (1290, 264, 3)])
+@pytest.mark.parametrize("V,rank,b", [(77, 8, 16), (9000, 72, 5), (1290, 264, 3), (140000, 40, 1)])
 def test_markov_bounds_keep_the_pick(gpu, V, rank, b, kind):
     """Ranks and vocabularies off the tile sizes, and rows whose bounds say little: masked logits,
-    equal scores (more candidates than a workgroup keeps), infinities, values below the normal
-    range. The picks are the fp64 oracle's, bit for bit."""
+    equal scores (more candidates than a workgroup sums one by one, and than it keeps), infinities,
+    values below the normal range. The picks are the fp64 oracle's, bit for bit."""
     from snowllm_amd.draft_heads import MarkovHead
     _say(f"dspark markov bounds V={V} rank={rank} b={b} {kind}")
     block = 3
