@@ -835,184 +835,316 @@ __global__ void __launch_bounds__(WIDE_NT) wide_scatter(WideArgs a) {
 static_assert(VOCAB_MAX / WIDE_CHUNK <= WAVE, "one lane per bucketing workgroup");
 static_assert(WIDE_RUN * (WIDE_NT / WAVE) == 2 * WAVE, "two zero counts per lane");
 
-// Items too many for LDS (thousands of nearly equal probabilities): one workgroup sorts the
-// range. A bitmap of the range's indices in LDS gives them in ascending order (equal keys are
-// then done), and a stable radix sort of the key bits that differ follows, 8 bits per pass,
-// between the two item buffers. lds: 2^14 words.
-__device__ __attribute__((noinline)) void wide_sort_range(const WideArgs& a, int row, uint64_t* src,
-                                                          uint64_t* dst, int n, uint32_t* lds) {
-  constexpr int NW = WIDE_NT / WAVE;
-  __shared__ uint32_t s_w[NW], s_min, s_max;
-  const int t = threadIdx.x, lane = t & (WAVE - 1), w = t / WAVE;
-  const uint64_t below = (1ull << lane) - 1ull;
-  const float* x = a.dense + (int64_t)row * a.V;
-  const int words = (int)((a.V + 31) / 32);
+constexpr int WIDE_SUB = 2048, WIDE_SUB_MAX = 48;  // finer bins of a sort, most items of one
+constexpr int WIDE_SEG = 4 * WIDE_T;               // sorted positions of a workgroup of a long range
+constexpr int WIDE_ITEMS = WIDE_CAP / WIDE_NT;
+static_assert(WIDE_SEG <= WIDE_CAP, "a segment fits LDS");
+
+struct WideShared {
+  uint64_t it[WIDE_CAP];
+  uint32_t bin[WIDE_SUB + 1], w[WIDE_NT / WAVE];
+  uint32_t most;
+};
+
+// Sorts n <= WIDE_CAP items, WIDE_ITEMS per thread (thread t: t, t + WIDE_NT, ...): counted into
+// WIDE_SUB bins (bin(item): ascending with the item), laid out bin by bin in LDS, and each item's
+// place is its bin's start plus the smaller items of its bin; where a bin holds many, a bitonic
+// sort. emit(place, item). sh.bin and sh.most are cleared, every thread past a barrier since.
+template <class Bin, class Emit>
+__device__ __forceinline__ void wide_sort_items(WideShared& sh, const uint64_t (&it)[WIDE_ITEMS],
+                                                int n, Bin&& bin, Emit&& emit) {
+  const int t = threadIdx.x;
+  uint32_t at[WIDE_ITEMS];
+#pragma unroll
+  for (int j = 0; j < WIDE_ITEMS; ++j) {
+    if (j * WIDE_NT >= n) break;
+    if (j * WIDE_NT + t < n) at[j] = atomicAdd(&sh.bin[bin(it[j])], 1u);
+  }
   __syncthreads();
-  for (int i = t; i < words; i += WIDE_NT) lds[i] = 0u;
-  if (t == 0) s_min = 0xffffffffu, s_max = 0u;
+  {
+    // bin starts: two bins per thread, and the fullest bin
+    const uint32_t c0 = sh.bin[2 * t], c1 = sh.bin[2 * t + 1];
+    uint32_t incl = c0 + c1, most = c0 > c1 ? c0 : c1;
+#pragma unroll
+    for (int d = 1; d < WAVE; d <<= 1) {
+      const uint32_t o = (uint32_t)__shfl_up((int)incl, d, WAVE);
+      if ((t & (WAVE - 1)) >= d) incl += o;
+    }
+    most = wave_max(most);
+    if ((t & (WAVE - 1)) == WAVE - 1) {
+      sh.w[t / WAVE] = incl;
+      atomicMax(&sh.most, most);
+    }
+    __syncthreads();
+    uint32_t pre = incl - c0 - c1;
+    for (int i = 0; i < t / WAVE; ++i) pre += sh.w[i];
+    sh.bin[2 * t] = pre;
+    sh.bin[2 * t + 1] = pre + c0;
+    if (t == 0) sh.bin[WIDE_SUB] = (uint32_t)n;
+  }
+  __syncthreads();
+  if (sh.most <= WIDE_SUB_MAX) {  // uniform
+#pragma unroll
+    for (int j = 0; j < WIDE_ITEMS; ++j) {
+      if (j * WIDE_NT >= n) break;
+      if (j * WIDE_NT + t < n) sh.it[sh.bin[bin(it[j])] + at[j]] = it[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < WIDE_ITEMS; ++j) {
+      if (j * WIDE_NT >= n) break;
+      if (j * WIDE_NT + t < n) {
+        const uint32_t b = bin(it[j]);
+        uint32_t pos = sh.bin[b];
+        const uint32_t end = sh.bin[b + 1];
+        for (uint32_t u = sh.bin[b]; u < end; ++u) pos += sh.it[u] < it[j];
+        emit((int)pos, it[j]);
+      }
+    }
+    return;
+  }
+  int n2 = 64;
+  while (n2 < n) n2 <<= 1;
+#pragma unroll
+  for (int j = 0; j < WIDE_ITEMS; ++j) {
+    if (j * WIDE_NT >= n) break;
+    if (j * WIDE_NT + t < n) sh.it[j * WIDE_NT + t] = it[j];
+  }
+  for (int i = n + t; i < n2; i += WIDE_NT) sh.it[i] = ~0ull;
+  __syncthreads();
+  // bitonic sort, ascending (items are unique)
+  for (int size = 2; size <= n2; size <<= 1) {
+    for (int stride = size >> 1; stride > 0; stride >>= 1) {
+      for (int e = t; e < n2 / 2; e += WIDE_NT) {
+        const int i = ((e & ~(stride - 1)) << 1) | (e & (stride - 1)), j = i | stride;
+        const uint64_t x = sh.it[i], y = sh.it[j];
+        if (((i & size) == 0) ? x > y : x < y) {
+          sh.it[i] = y;
+          sh.it[j] = x;
+        }
+      }
+      __syncthreads();
+    }
+  }
+  for (int i = t; i < n; i += WIDE_NT) emit(i, sh.it[i]);
+}
+
+// Sorted positions [r0, r_end) of a range of n items that LDS does not hold (thousands of nearly
+// equal probabilities); its other positions are other workgroups'. An item counts as
+// (key - least key) 2^vb + index, so equal keys spread by their index. Each round counts the
+// items of a value interval into 4096 bins and takes the bins from r0's on that fit LDS together,
+// or goes into r0's bin alone while that one does not; then those items are read into LDS and
+// sorted. Ends: a bin's interval is at most 2^-11 of its parent's and bins of one value hold one
+// item, and each turn of the outer loop places r0 at least.
+__device__ __attribute__((noinline)) void wide_sort_segment(const WideArgs& a, const uint64_t* src,
+                                                            uint64_t* dst, int n, int r0, int r_end,
+                                                            WideShared& sh) {
+  constexpr int HB = 4096, PER = HB / WIDE_NT, UN = 8;
+  __shared__ uint32_t s_kmin, s_kmax, s_first, s_last, s_start, s_stop, s_end, s_cnt;
+  uint32_t* h = (uint32_t*)sh.it;  // [HB]: the counts and the items take turns
+  const int t = threadIdx.x, lane = t & (WAVE - 1), w = t / WAVE;
+  auto each = [&](auto&& f) {  // every item, UN loads in flight
+    for (int i0 = t; i0 < n; i0 += WIDE_NT * UN) {
+      uint64_t x[UN];
+#pragma unroll
+      for (int u = 0; u < UN; ++u) x[u] = src[i0 + u * WIDE_NT < n ? i0 + u * WIDE_NT : n - 1];
+#pragma unroll
+      for (int u = 0; u < UN; ++u)
+        if (i0 + u * WIDE_NT < n) f(x[u]);
+    }
+  };
+  // one add for the lanes of the first active lane's bin, twice: a wave's items often share a bin
+  // (equal keys come with neighbouring indices), and adds on one address go one after another
+  auto count = [&](uint32_t b) {
+    const uint32_t b0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)b);
+    const uint64_t m0 = __ballot(b == b0);
+    if (lane == (int)__builtin_ctzll(m0)) atomicAdd(&h[b0], (uint32_t)__popcll(m0));
+    if (b != b0) {
+      const uint32_t b1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)b);
+      const uint64_t m1 = __ballot(b == b1);
+      if (lane == (int)__builtin_ctzll(m1)) atomicAdd(&h[b1], (uint32_t)__popcll(m1));
+      if (b != b1) atomicAdd(&h[b], 1u);
+    }
+  };
+  __syncthreads();
+  if (t == 0) s_kmin = 0xffffffffu, s_kmax = 0u;
   __syncthreads();
   uint32_t kmin = 0xffffffffu, kmax = 0u;
-  for (int i = t; i < n; i += WIDE_NT) {
-    const uint64_t it = src[i];
-    const uint32_t key = (uint32_t)(it >> 32), at = (uint32_t)it;
+  each([&](uint64_t x) {
+    const uint32_t key = (uint32_t)(x >> 32);
     kmin = key < kmin ? key : kmin;
     kmax = key > kmax ? key : kmax;
-    atomicOr(&lds[at >> 5], 1u << (at & 31));
-  }
+  });
   kmin = ~wave_max(~kmin), kmax = wave_max(kmax);
   if (lane == 0) {
-    atomicMin(&s_min, kmin);
-    atomicMax(&s_max, kmax);
+    atomicMin(&s_kmin, kmin);
+    atomicMax(&s_kmax, kmax);
   }
   __syncthreads();
-  kmin = s_min;
-  const uint32_t span = s_max - kmin;
-  const int passes = span ? (32 - __builtin_clz(span) + 7) / 8 : 0;
-  // the items in index order, where an even or odd number of passes ends in dst
-  const int per = (words + WIDE_NT - 1) / WIDE_NT;
-  uint32_t cnt = 0;
-  for (int i = t * per; i < t * per + per && i < words; ++i) cnt += __popc(lds[i]);
-  uint32_t incl = cnt;
+  kmin = s_kmin;
+  const int vb = 32 - __builtin_clz((uint32_t)a.V - 1u);  // (V > 1024)
+  const uint64_t top = ((uint64_t)(s_kmax - kmin) << vb) | ((1ull << vb) - 1ull);
+  auto value = [&](uint64_t x) {
+    return ((uint64_t)((uint32_t)(x >> 32) - kmin) << vb) | (uint64_t)(uint32_t)x;
+  };
+  while (r0 < r_end) {  // uniform, as every branch on it below
+    uint64_t vlo = 0, vhi = top;  // the interval, and the items below it
+    int before = 0, r1 = r_end;
+    for (;;) {
+      const uint64_t span = vhi - vlo;
+      const int bits = span ? 64 - (int)__builtin_clzll(span) : 0;
+      const int shift = bits > 12 ? bits - 12 : 0;  // span >> shift < HB
+      for (int i = t; i < HB; i += WIDE_NT) h[i] = 0u;
+      if (t == 0) s_last = 0u, s_end = 0u, s_cnt = 0u;
+      __syncthreads();
+      each([&](uint64_t x) {
+        const uint64_t v = value(x);
+        if (v >= vlo && v <= vhi) count((uint32_t)((v - vlo) >> shift));
+      });
+      __syncthreads();
+      uint32_t c[PER], run = 0;
 #pragma unroll
-  for (int d = 1; d < WAVE; d <<= 1) {
-    const uint32_t o = (uint32_t)__shfl_up((int)incl, d, WAVE);
-    if (lane >= d) incl += o;
-  }
-  if (lane == WAVE - 1) s_w[w] = incl;
-  __syncthreads();
-  uint32_t pos = incl - cnt;
-  for (int i = 0; i < w; ++i) pos += s_w[i];
-  uint64_t* from = passes & 1 ? src : dst;
-  uint64_t* to = passes & 1 ? dst : src;
-  for (int i = t * per; i < t * per + per && i < words; ++i)
-    for (uint32_t m = lds[i]; m; m &= m - 1) {
-      const int at = i * 32 + __builtin_ctz(m);
-      from[pos++] = wide_item(x[at], at);
-    }
-  uint32_t* base = lds;                 // [256]
-  uint32_t* wcnt = lds + 256;           // [NW][256]
-  for (int pass = 0; pass < passes; ++pass) {
-    const int shift = 8 * pass;
-    auto digit = [&](uint64_t it) { return (((uint32_t)(it >> 32) - kmin) >> shift) & 255u; };
-    __syncthreads();
-    for (int i = t; i < 256 * (NW + 1); i += WIDE_NT) lds[i] = 0u;
-    __syncthreads();
-    for (int i = t; i < n; i += WIDE_NT) atomicAdd(&base[digit(from[i])], 1u);
-    __syncthreads();
-    if (w == 0) {  // exclusive prefix, four digits per lane
-      uint32_t v[4], s = 0;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = base[lane * 4 + i], s += v[i];
-      uint32_t in = s;
+      for (int i = 0; i < PER; ++i) c[i] = h[t * PER + i], run += c[i];
+      uint32_t incl = run;
 #pragma unroll
       for (int d = 1; d < WAVE; d <<= 1) {
-        const uint32_t o = (uint32_t)__shfl_up((int)in, d, WAVE);
-        if (lane >= d) in += o;
+        const uint32_t o = (uint32_t)__shfl_up((int)incl, d, WAVE);
+        if (lane >= d) incl += o;
       }
-      uint32_t pre = in - s;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        base[lane * 4 + i] = pre;
-        pre += v[i];
-      }
-    }
-    __syncthreads();
-    for (int i0 = 0; i0 < n; i0 += WIDE_NT) {
-      const bool live = i0 + t < n;
-      const uint64_t it = from[live ? i0 + t : n - 1];
-      const uint32_t d = digit(it);
-      uint64_t same = __ballot(live);
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const uint64_t ones = __ballot((d >> q) & 1u);
-        same &= ((d >> q) & 1u) ? ones : ~ones;
-      }
-      const uint32_t rank = (uint32_t)__popcll(same & below);
-      if (live && rank == 0) wcnt[w * 256 + d] = (uint32_t)__popcll(same);
+      if (lane == WAVE - 1) sh.w[w] = incl;
       __syncthreads();
-      if (live) {
-        uint32_t p = base[d] + rank;
-        for (int ww = 0; ww < w; ++ww) p += wcnt[ww * 256 + d];
-        to[p] = it;
+      uint32_t first = (uint32_t)before + incl - run;  // the rank where this thread's bins start
+      for (int i = 0; i < w; ++i) first += sh.w[i];
+      uint32_t pos = first;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        if (pos <= (uint32_t)r0 && (uint32_t)r0 < pos + c[i])
+          s_first = (uint32_t)(t * PER + i), s_start = pos, s_stop = pos + c[i];  // one bin
+        pos += c[i];
       }
       __syncthreads();
-      if (t < 256) {
-        uint32_t tot = 0;
-        for (int ww = 0; ww < NW; ++ww) {
-          tot += wcnt[ww * 256 + t];
-          wcnt[ww * 256 + t] = 0u;
+      const uint32_t f = s_first, start = s_start, stop = s_stop;
+      if (stop - start > (uint32_t)WIDE_CAP) {  // (shift > 0: one value is one item)
+        vlo += (uint64_t)f << shift;
+        const uint64_t last = vlo + (1ull << shift) - 1ull;
+        vhi = last < vhi ? last : vhi;
+        before = (int)start;
+        r1 = (int)stop < r1 ? (int)stop : r1;
+        __syncthreads();
+        continue;
+      }
+      pos = first;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const uint32_t b = (uint32_t)(t * PER + i);
+        if (b >= f && c[i] && pos < (uint32_t)r1 && pos + c[i] - start <= (uint32_t)WIDE_CAP) {
+          atomicMax(&s_last, b);
+          atomicMax(&s_end, pos + c[i]);
         }
-        base[t] += tot;
+        pos += c[i];
+      }
+      __syncthreads();  // (h is read: the items may take its place)
+      const uint64_t clo = vlo + ((uint64_t)f << shift);
+      uint64_t chi = vlo + (((uint64_t)s_last + 1ull) << shift) - 1ull;
+      chi = chi < vhi ? chi : vhi;
+      const int end = (int)s_end, m = end - (int)start, done = end < r1 ? end : r1;
+      each([&](uint64_t x) {
+        const uint64_t v = value(x);
+        if (v >= clo && v <= chi) sh.it[atomicAdd(&s_cnt, 1u)] = x;
+      });
+      for (int i = t; i < WIDE_SUB; i += WIDE_NT) sh.bin[i] = 0u;
+      if (t == 0) sh.most = 0u;
+      __syncthreads();
+      uint64_t it[WIDE_ITEMS];
+#pragma unroll
+      for (int j = 0; j < WIDE_ITEMS; ++j) {
+        if (j * WIDE_NT >= m) break;
+        it[j] = sh.it[j * WIDE_NT + t < m ? j * WIDE_NT + t : m - 1];
       }
       __syncthreads();
+      const int cbits = chi > clo ? 64 - (int)__builtin_clzll(chi - clo) : 0;
+      const int cs = cbits > 11 ? cbits - 11 : 0;  // (chi - clo) >> cs < WIDE_SUB
+      wide_sort_items(sh, it, m, [&](uint64_t x) { return (uint32_t)((value(x) - clo) >> cs); },
+                      [&](int place, uint64_t x) {
+                        const int r = (int)start + place;
+                        if (r >= r0 && r < done) dst[r] = x;
+                      });
+      r0 = done;
+      __syncthreads();
+      break;
     }
-    uint64_t* o = from;
-    from = to;
-    to = o;
   }
 }
-static_assert(VOCAB_MAX / 32 <= WIDE_CAP * 2, "the range's bitmap fits the items' LDS");
 
-// The buckets that start in positions [WIDE_T w, WIDE_T (w + 1)), sorted: workgroup w of a row.
-// The items are counted into WIDE_SUB finer bins of their key range (a few per bin), laid out
-// bin by bin in LDS, and each item's place is its bin's start plus the smaller items of its bin.
-// Where a bin holds many (equal or clustered probabilities) a bitonic sort takes its place.
-constexpr int WIDE_SUB = 2048, WIDE_SUB_MAX = 48;
-__global__ void __launch_bounds__(WIDE_NT) wide_sort(WideArgs a) {
-  __shared__ uint64_t s_it[WIDE_CAP];
-  __shared__ uint32_t s_bin[WIDE_SUB + 1], s_w[WIDE_NT / WAVE];
-  __shared__ uint32_t s_lo, s_hi, s_min, s_max, s_most;
-  constexpr int ITEMS = WIDE_CAP / WIDE_NT;
-  const int row = blockIdx.y, t = threadIdx.x;
+// The buckets that start in positions [WIDE_T w, WIDE_T (w + 1)), sorted: workgroup w of a row. A
+// bucket that LDS may not hold beside the others (equal or nearly equal probabilities) is sorted in
+// segments of WIDE_SEG positions by this workgroup and every fourth of those that follow within it.
+// MI355X, 151,936 logits, us for the launches of the lists, with a four-pass radix sort / one
+// workgroup for such a bucket / now. 9 rows of standard deviation 3: 219 / 88 / 88, 0.05: 226 / 207
+// / 184, 0.01: 227 / 478 / 188, 0.001: 232 / 1349 / 298, all equal: 207 / 438 / 251, all but
+// one equal: 204 / 1933 / 262.
+__global__ void __launch_bounds__(WIDE_NT) __attribute__((amdgpu_waves_per_eu(8)))
+wide_sort(WideArgs a) {
+  __shared__ WideShared sh;
+  __shared__ uint32_t s_lo, s_hi, s_prev, s_last, s_min, s_max;
+  const int row = blockIdx.y, t = threadIdx.x, lane = t & (WAVE - 1);
   int64_t k;
   bool nuc;
   if (!wide_row(a, row, &k, &nuc)) return;
   const int bins = 1 << a.bins_log;
   const uint32_t* start = a.hist + (int64_t)row * 256 * a.C + bins;
   const uint32_t from = (uint32_t)blockIdx.x * WIDE_T, to = from + WIDE_T;
-  if (t == 0) s_lo = s_hi = (uint32_t)a.V;
+  if (t == 0) s_lo = s_hi = (uint32_t)a.V, s_prev = s_last = 0u;
   __syncthreads();
   constexpr int PER = WIDE_BINS / WIDE_NT;
-  uint32_t lo = 0xffffffffu, hi = 0xffffffffu;
+  uint32_t lo = 0xffffffffu, hi = 0xffffffffu, prev = 0u, last = 0u;
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int at = t + i * WIDE_NT;
     const uint32_t s = at < bins ? start[at] : 0xffffffffu;
     if (s >= from && s < lo) lo = s;
     if (s >= to && s < hi) hi = s;
+    if (s < from && s > prev) prev = s;
+    if (s < to && s > last) last = s;
   }
-  lo = ~wave_max(~lo);
-  hi = ~wave_max(~hi);
-  if ((t & (WAVE - 1)) == 0) {
+  lo = wave_min_u32_dpp(lo);
+  hi = wave_min_u32_dpp(hi);
+  prev = wave_max_u32_dpp(prev);
+  last = wave_max_u32_dpp(last);
+  if (lane == 0) {
     atomicMin(&s_lo, lo);
     atomicMin(&s_hi, hi);
+    atomicMax(&s_prev, prev);
+    atomicMax(&s_last, last);
   }
   __syncthreads();
-  lo = s_lo, hi = s_hi;
+  lo = s_lo, hi = s_hi, prev = s_prev, last = s_last;
   // the range without the zeros, which are in their places: what lies before and behind them
   const uint32_t z0 = start[bins - 2], z1 = start[bins - 1];
+  auto is_long = [&](uint32_t b0, uint32_t b1) {  // a bucket, not the zeros'
+    return b1 > b0 && b1 - b0 > WIDE_CAP - WIDE_T && !(b0 == z0 && z1 > z0);
+  };
+  const bool own_long = last >= from && is_long(last, hi);       // the last bucket from here
+  const bool other_long = from > 0 && is_long(prev, lo) && lo > from;  // one from before
+  const uint32_t end = own_long ? last : hi;
   for (int side = 0; side < 2; ++side) {
-    const uint32_t b0 = side ? (lo > z1 ? lo : z1) : lo, b1 = side ? hi : (hi < z0 ? hi : z0);
+    const uint32_t b0 = side ? (lo > z1 ? lo : z1) : lo, b1 = side ? end : (end < z0 ? end : z0);
     if (b0 >= b1) continue;  // uniform
-    uint64_t* src = a.items[1] + (int64_t)row * a.V + b0;
+    const int n = (int)(b1 - b0);  // at most WIDE_T - 1 + (WIDE_CAP - WIDE_T)
+    const uint64_t* src = a.items[1] + (int64_t)row * a.V + b0;
     uint64_t* dst = a.items[0] + (int64_t)row * a.V + b0;
-    const int n = (int)(b1 - b0);
-    if (n > WIDE_CAP) {
-      wide_sort_range(a, row, src, dst, n, (uint32_t*)s_it);
-      continue;
-    }
-    uint64_t it[ITEMS];
+    uint64_t it[WIDE_ITEMS];
 #pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
+    for (int j = 0; j < WIDE_ITEMS; ++j) {
       if (j * WIDE_NT >= n) break;  // uniform
       it[j] = src[j * WIDE_NT + t < n ? j * WIDE_NT + t : n - 1];
     }
     __syncthreads();
-    if (t == 0) s_min = 0xffffffffu, s_max = 0u, s_most = 0u;
-    for (int i = t; i < WIDE_SUB; i += WIDE_NT) s_bin[i] = 0u;
+    if (t == 0) s_min = 0xffffffffu, s_max = 0u, sh.most = 0u;
+    for (int i = t; i < WIDE_SUB; i += WIDE_NT) sh.bin[i] = 0u;
     uint32_t kmin = 0xffffffffu, kmax = 0u;
 #pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
+    for (int j = 0; j < WIDE_ITEMS; ++j) {
       if (j * WIDE_NT >= n) break;
       const uint32_t key = (uint32_t)(it[j] >> 32);
       kmin = key < kmin ? key : kmin;
@@ -1020,7 +1152,7 @@ __global__ void __launch_bounds__(WIDE_NT) wide_sort(WideArgs a) {
     }
     kmin = ~wave_max(~kmin), kmax = wave_max(kmax);
     __syncthreads();
-    if ((t & (WAVE - 1)) == 0) {
+    if (lane == 0) {
       atomicMin(&s_min, kmin);
       atomicMax(&s_max, kmax);
     }
@@ -1028,81 +1160,20 @@ __global__ void __launch_bounds__(WIDE_NT) wide_sort(WideArgs a) {
     kmin = s_min;
     const uint32_t span = s_max - kmin;
     const int bits = span ? 32 - __builtin_clz(span) : 0;
-    const int sh = bits > 11 ? bits - 11 : 0;  // span >> sh < WIDE_SUB
-    uint32_t at[ITEMS];
-#pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
-      if (j * WIDE_NT >= n) break;
-      if (j * WIDE_NT + t < n) at[j] = atomicAdd(&s_bin[((uint32_t)(it[j] >> 32) - kmin) >> sh], 1u);
-    }
-    __syncthreads();
-    {
-      // bin starts: two bins per thread, and the fullest bin
-      const uint32_t c0 = s_bin[2 * t], c1 = s_bin[2 * t + 1];
-      uint32_t incl = c0 + c1, most = c0 > c1 ? c0 : c1;
-#pragma unroll
-      for (int d = 1; d < WAVE; d <<= 1) {
-        const uint32_t o = (uint32_t)__shfl_up((int)incl, d, WAVE);
-        if ((t & (WAVE - 1)) >= d) incl += o;
-      }
-      most = wave_max(most);
-      if ((t & (WAVE - 1)) == WAVE - 1) {
-        s_w[t / WAVE] = incl;
-        atomicMax(&s_most, most);
-      }
-      __syncthreads();
-      uint32_t pre = incl - c0 - c1;
-      for (int i = 0; i < t / WAVE; ++i) pre += s_w[i];
-      s_bin[2 * t] = pre;
-      s_bin[2 * t + 1] = pre + c0;
-      if (t == 0) s_bin[WIDE_SUB] = (uint32_t)n;
-    }
-    __syncthreads();
-    if (s_most <= WIDE_SUB_MAX) {  // uniform
-#pragma unroll
-      for (int j = 0; j < ITEMS; ++j) {
-        if (j * WIDE_NT >= n) break;
-        if (j * WIDE_NT + t < n)
-          s_it[s_bin[((uint32_t)(it[j] >> 32) - kmin) >> sh] + at[j]] = it[j];
-      }
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < ITEMS; ++j) {
-        if (j * WIDE_NT >= n) break;
-        if (j * WIDE_NT + t < n) {
-          const uint32_t bin = ((uint32_t)(it[j] >> 32) - kmin) >> sh;
-          uint32_t pos = s_bin[bin];
-          const uint32_t end = s_bin[bin + 1];
-          for (uint32_t u = s_bin[bin]; u < end; ++u) pos += s_it[u] < it[j];
-          dst[pos] = it[j];
-        }
-      }
-      continue;
-    }
-    int n2 = 64;
-    while (n2 < n) n2 <<= 1;
-#pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
-      if (j * WIDE_NT >= n) break;
-      if (j * WIDE_NT + t < n) s_it[j * WIDE_NT + t] = it[j];
-    }
-    for (int i = n + t; i < n2; i += WIDE_NT) s_it[i] = ~0ull;
-    __syncthreads();
-    // bitonic sort, ascending (items are unique)
-    for (int size = 2; size <= n2; size <<= 1) {
-      for (int stride = size >> 1; stride > 0; stride >>= 1) {
-        for (int e = t; e < n2 / 2; e += WIDE_NT) {
-          const int i = ((e & ~(stride - 1)) << 1) | (e & (stride - 1)), j = i | stride;
-          const uint64_t x = s_it[i], y = s_it[j];
-          if (((i & size) == 0) ? x > y : x < y) {
-            s_it[i] = y;
-            s_it[j] = x;
-          }
-        }
-        __syncthreads();
-      }
-    }
-    for (int i = t; i < n; i += WIDE_NT) dst[i] = s_it[i];
+    const int shift = bits > 11 ? bits - 11 : 0;  // span >> shift < WIDE_SUB
+    wide_sort_items(sh, it, n,
+                    [&](uint64_t x) { return ((uint32_t)(x >> 32) - kmin) >> shift; },
+                    [&](int place, uint64_t x) { dst[place] = x; });
+  }
+  if (__builtin_expect(!own_long && !other_long, 1)) return;  // uniform
+  for (int job = 0; job < 2; ++job) {
+    if (!(job ? other_long : own_long)) continue;
+    const uint32_t b0 = job ? prev : last, b1 = job ? lo : hi;
+    const int n = (int)(b1 - b0), w = job ? (int)(blockIdx.x - b0 / WIDE_T) : 0;
+    const int seg = w / 4 * WIDE_SEG;
+    if (w % 4 != 0 || seg >= n) continue;
+    wide_sort_segment(a, a.items[1] + (int64_t)row * a.V + b0, a.items[0] + (int64_t)row * a.V + b0,
+                      n, seg, seg + WIDE_SEG < n ? seg + WIDE_SEG : n, sh);
   }
 }
 

@@ -29,9 +29,12 @@ def _rows(V, seed):
 
 
 def _check(V, top_k, top_p, seed):
+    _check_rows(_rows(V, seed), top_k, top_p)
+
+
+def _check_rows(x, top_k, top_p):
     from snowllm_amd import ops
-    x = _rows(V, seed)
-    n = x.shape[0]
+    n, V = x.shape
     width = max(min(k, V) if k > 0 else V for k in top_k)
     k = torch.tensor(top_k, dtype=torch.int32)
     p = torch.tensor(top_p)
@@ -66,6 +69,25 @@ def test_wide_lists(gpu, V):
     """The whole vocabulary with top-p, widths between, short lists beside them."""
     _check(V, [0, V, 0, 1025, 0, 0, 0], [0.9, 0.5, 0.95, 1.0, 0.8, 0.3, 0.999], V)
     _check(V, [1026, 20, V - 1, 0, 0, 1050, 7], [0.9, 0.5, 1.0, 0.9, 1.0, 0.95, 1.0], V + 1)
+
+
+@pytest.mark.parametrize("V", [12000, 50257, 151936])
+def test_wide_lists_of_crowded_rows(gpu, V):
+    """More nearly equal probabilities than a workgroup sorts in LDS, so that several share a range:
+    distinct ones in one bucket and in neighbouring ones, a few values many times each, two heavy
+    values, one value, and one beside a peak."""
+    g = torch.Generator().manual_seed(V)
+    x = torch.randn(8, V, generator=g)
+    x[0] *= 0.001
+    x[1] *= 0.01
+    x[2] *= 0.0001
+    x[3] = (x[3] * 2).round() * 0.003
+    x[4] = torch.where(torch.rand(V, generator=g) < 0.5, 0.0, -0.004)
+    x[5] = 1.25
+    x[6] = torch.where(torch.arange(V) == V // 3, 40.0, 0.0)
+    x[7] = torch.where(torch.rand(V, generator=g) < 0.7, 1.0, 0.05 * x[7])
+    _check_rows(x, [0] * 8, [0.9, 0.5, 0.95, 0.3, 0.8, 0.6, 0.999, 0.7])
+    _check_rows(x, [V - 5, 1500, V, 9000, 0, 2000, 11000, 0], [1.0, 0.9, 0.2, 1.0, 0.99, 1.0, 0.9, 1.0])
 
 
 @pytest.mark.parametrize("p_width,q_width", [(1, 16), (20, 16), (4096, 16), (4097, 70), (9000, 9000)])
