@@ -90,6 +90,19 @@ def test_wide_lists_of_crowded_rows(gpu, V):
     _check_rows(x, [V - 5, 1500, V, 9000, 0, 2000, 11000, 0], [1.0, 0.9, 0.2, 1.0, 0.99, 1.0, 0.9, 1.0])
 
 
+@pytest.mark.parametrize("k", [200, 1000])
+def test_short_lists_of_many_candidates(gpu, k):
+    """Large distinct values in a few threads' words: more elements lie above the threshold than LDS
+    holds, and the exact selection takes over (k at or below 256 keeps one key per thread, two
+    above)."""
+    V = 151936
+    g = torch.Generator().manual_seed(k)
+    x = torch.randn(2, V, generator=g)
+    heavy = (torch.arange(V) // 4) % 1024 < 150
+    x = torch.where(heavy, x.abs() + 6, x)
+    _check_rows(x, [k, k], [1.0, 0.9])
+
+
 @pytest.mark.parametrize("p_width,q_width", [(1, 16), (20, 16), (4096, 16), (4097, 70), (9000, 9000)])
 def test_reject_searches(gpu, p_width, q_width):
     """Draft tokens in unordered lists, present, absent and repeated (their sum), with stale
@@ -119,6 +132,32 @@ def test_reject_searches(gpu, p_width, q_width):
     for u in (torch.rand(b, k + 1, generator=g), torch.rand(b, k + 1, generator=g) * 0.02,
               torch.zeros(b, k + 1)):
         print(f"reject p_width={p_width} q_width={q_width}", flush=True)
+        ops.dflash.reject(*[x.cuda() for x in args], u.cuda(), out, acc)
+        want, wacc = A.reject(*[x.numpy() for x in args], u.numpy())
+        assert np.array_equal(acc.cpu().numpy(), wacc)
+        assert np.array_equal(out.cpu().numpy(), want)
+
+
+def test_reject_of_a_block_past_the_search_array(gpu):
+    """A block of more draft rows than the array of matches holds, with target lists wider than a
+    chunk: the waves search the lists themselves."""
+    from snowllm_amd import ops
+    k, p_width, q_width = 2060, 4097, 16
+    g = torch.Generator().manual_seed(5)
+    print(f"reject block={k} p_width={p_width}", flush=True)
+    p = torch.rand(k + 1, p_width, generator=g)
+    p /= p.sum(-1, keepdim=True)
+    ids = (torch.arange(p_width) * 5 + torch.arange(k + 1).unsqueeze(1) * 3) % 30000
+    drafts = ids[torch.arange(k), torch.randint(0, p_width, (k,), generator=g)].view(1, k).clone()
+    cand = torch.randint(0, 30000, (1, k, q_width), generator=g)
+    cand[0, :, 3] = drafts[0]
+    q = torch.rand(1, k, q_width, generator=g) * 1e-4
+    one = torch.ones(1, dtype=torch.int32)
+    args = [p, ids.contiguous(), drafts, cand, q, one * 0, one]
+    out = torch.empty(1, k + 1, dtype=torch.int64, device="cuda")
+    acc = torch.empty(1, dtype=torch.int64, device="cuda")
+    u = torch.rand(1, k + 1, generator=g)
+    for u in (u * 1e-3, u, u * 0.0):
         ops.dflash.reject(*[x.cuda() for x in args], u.cuda(), out, acc)
         want, wacc = A.reject(*[x.numpy() for x in args], u.numpy())
         assert np.array_equal(acc.cpu().numpy(), wacc)
