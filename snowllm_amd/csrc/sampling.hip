@@ -126,12 +126,6 @@ __global__ void __launch_bounds__(NT) softmax_max(const float* __restrict__ logi
     tail.max_keys[row * C + c] = ord_key(__fdiv_rn(ord_key_to_float(best), T));
 }
 
-__device__ __forceinline__ float row_max_from_keys(const uint32_t* keys, int C) {
-  uint32_t m = 0;
-  for (int c = 0; c < C; ++c) m = keys[c] > m ? keys[c] : m;
-  return ord_key_to_float(m);
-}
-
 __global__ void __launch_bounds__(NT) softmax_exp(const float* __restrict__ logits, int64_t V,
                                                   const float* __restrict__ temperature,
                                                   float* __restrict__ dense, SoftmaxTail tail,
@@ -1900,7 +1894,7 @@ SV_API int snowllm_sampling_penalties(float* logits, const int64_t* ids, const i
 }
 
 // Lists wider than TOPK_MAX add the wide-list sort: two [batch, vocab] u64 item buffers, the
-// per-pass chunk histograms and the per-row sums.
+// buckets' counts and starts, and two sums per chunk of each row.
 namespace {
 size_t lists_bytes(int64_t batch, int64_t vocab, int64_t width) {
   const int64_t C = chunks_of(vocab);
@@ -1946,7 +1940,7 @@ SV_API int64_t snowllm_sampling_workspace_bytes(int64_t batch, int64_t vocab, in
   if (width > TOPK_MAX) {
     const int64_t C = chunks_of(vocab);
     bytes += 2 * align256((size_t)batch * vocab * 8) + align256((size_t)batch * 256 * C * 4) +
-             2 * align256((size_t)batch * C * 8) + align256((size_t)batch * 16);
+             2 * align256((size_t)batch * C * 8);
   }
   return (int64_t)bytes;
 }
