@@ -454,9 +454,8 @@ def bench_step(args, name):
             n0, m.moe_slots[0], c.experts, H, F),
             slots0 * (q4k_bytes(2 * F, H) + q4k_bytes(H, F)))
     else:
-        n0 = m.row_chunks[0][1]
-        per_launch("gate_up_swiglu", lambda i: Lops.gate_up_swiglu(
-            c.ffn_fmt, Lw[i].gu[0], Lw[i].gu[1], m.ws_h2, m.act[:n0], n0, c.ffn, H),
+        per_launch("gate_up_swiglu", lambda i: Lops.gate_up_swiglu_rows(
+            c.ffn_fmt, Lw[i].gu[0], Lw[i].gu[1], m.ws_h2, m.act, R, c.ffn, H),
             q4k_bytes(2 * c.ffn, H))
     if sel is not None:
         us = timed_graph(lambda: acc.propose(), 5, stream) * 1e3

@@ -240,18 +240,15 @@ class VerifyModel:
         torch.cuda.synchronize()
         self.head_wt = Lops.WT_F16   # or WT_BF16, or HEAD_KQUANT with self.head_fmt
         self.head_fmt = 0
-        # MoE layers: post-attention norm, router and routing/plan in one launch where the
-        # fused kernel takes the shape (False: the three separate launches, the same bits)
-        # the MoE runs on row chunks (the fused router on chunks whose rows fit its LDS); the
-        # other layers' launches take every row
+        # the MoE runs on chunks of rows, every other launch takes all of them
         M = batch * c.block
         self.rows = M
-        self.row_chunks = [(r0, min(16, M - r0)) for r0 in range(0, M, 16)]
         # one MoE plan per 64 rows (an expert with more than 16 of them takes a slot per 16),
         # so each expert's weights are read once per 16 of its rows across the whole batch
         R = Lops.MOE_MAX_ROWS
         self.moe_chunks = [(r0, min(R, M - r0)) for r0 in range(0, M, R)]
-        # norm + router + routing/plan in one launch holds up to 16 rows
+        # post-attention norm, router and routing/plan in one launch where the fused kernel takes
+        # the shape, up to 16 rows (False: the three separate launches, the same bits)
         chunk = max(n for _, n in self.moe_chunks)
         self.fuse_router = bool(c.moe and chunk <= 16 and c.hidden % 512 == 0 and
                                 c.hidden <= 4096 and chunk * (c.hidden + 8) * 2 <= 131072 and
