@@ -217,16 +217,19 @@ __global__ void __launch_bounds__(NW * 64) dense_gemv(const u32x4* __restrict__ 
     vx = r < rows ? (uint32_t)(r * K * 2 + kq * 16) : 0x80000000u;
   }
   floatx4 acc[NTILE];
+  uint32_t wt0[NTILE];  // (a tile past the last: the last one again, not written)
 #pragma unroll
-  for (int t = 0; t < NTILE; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < NTILE; ++t) {
+    acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    wt0[t] = (uint32_t)((t < own ? t : own - 1) * S * 8 * 64 * 16);
+  }
   for (int s = wv; s < S; s += NW) {
     u32x4 wb[NTILE][8];
 #pragma unroll
     for (int t = 0; t < NTILE; ++t)
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        wb[t][j] = bload4(wr, lane * 16,
-                          (uint32_t)((((t < own ? t : own - 1) * S + s) * 8 + j) * 64 * 16));
+        wb[t][j] = bload4(wr, lane * 16, wt0[t] + (uint32_t)((s * 8 + j) * 64 * 16));
     u32x4 xa[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -273,16 +276,22 @@ __global__ void __launch_bounds__(NW * 64) dense_gemv(const u32x4* __restrict__ 
 // per superblock, the same sums over a wave's superblocks and over the waves). Both operands
 // stream one 32-wide k-step at a time, the activations DX and the weights DW steps ahead (rings
 // in registers); the rows' scales wait in LDS for the end of their superblock. Loads past a
-// wave's last superblock go out at out-of-range offsets and touch no memory. Bound: HBM, the
-// weights' bytes (nt loads, so that they do not displace the activations from L2), up to
-// about 128 rows; matrix instructions past that.
+// wave's last superblock go out at out-of-range offsets and touch no memory. Bound: the weights'
+// bytes from HBM (nt loads, so that they do not displace the activations from L2) at two row
+// tiles; from there on L2, which every workgroup reads the activations from once per 32 columns:
+// 108 rows of a 151,936 x 4096 bf16 head read 5.6 GB in 447 us, 12.6 TB/s, with the vector units
+// 9 % and the matrix units about 25 % busy.
+// Two row tiles need few enough registers for two workgroups a CU (one, before): 151,936 x 2048
+// fp16 at 24 rows 134 -> 113 us, 151,936 x 4096 bf16 268 -> 244; rings
+// twice as deep instead: 150 us.
 // MI355X, 151,936 x 4096 fp16, us (four row tiles per workgroup, weights loaded a superblock at
 // a time, before): 36 rows 331 -> 300, 108 rows 710 -> 449, 256 rows 1503 -> 978; x 2048 bf16,
 // 108 rows 533 -> 378.
 // Two row groups (more than 8 row tiles) take the same columns 8 apart in dispatch order, so that
 // both land on one XCD and the second's weights come from its L2.
 template <int WT, int NT, int NW, int MT>
-__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ void __launch_bounds__(NW * 64)
+    __attribute__((amdgpu_waves_per_eu(MT == 2 ? 4 : 2, MT == 2 ? 4 : 2)))
 dense_gemv_wide(const u32x4* __restrict__ w, const void* __restrict__ act, void* __restrict__ c,
                 int M, int N, int S, int c_bf16, size_t tile_bytes, int groups) {
   constexpr int DX = 2, DW = MT == 8 && WT == WT_F16 ? 2 : 4;  // (there two spill six registers already)
@@ -1573,17 +1582,21 @@ int launch_dense(const void* w, const void* act, void* c, int M, int N, int S, i
   const int row_tiles = (M + TILE_M - 1) / TILE_M;
   const size_t tb = xprep_tile_bytes(S);
   const int blocks = (tiles + NTILE - 1) / NTILE;
-  if (row_tiles == 1 || blocks < 64) {
+  const int wide = (tiles + 1) / 2;
+  if (row_tiles == 1 || blocks < 64 || (WT == WT_BF16 && row_tiles == 2 && wide <= 128)) {
     // one row tile per workgroup: a narrow output (the router's 17 tiles) then still has
-    // workgroups for several CUs (the same sums per row tile)
+    // workgroups for several CUs (the same sums per row tile). bf16 weights of up to 4096 columns
+    // at two row tiles likewise: 4096 x 4096 at 24 rows 13.6 us, 14.6 in one workgroup of both;
+    // 6144 x 4096 21.2 and 17.0
     hipLaunchKernelGGL((dense_gemv<WT, NTILE, NW>), dim3(blocks, row_tiles), dim3(NW * 64), 0, s,
                        (const u32x4*)w, act, c, M, N, S, c_bf16, tb);
     SV_CHECK_LAUNCH();
     return SV_OK;
   }
-  // every row tile in one workgroup up to DENSE_MT of them, two even groups above
-  const int groups = row_tiles > DENSE_MT ? 2 : 1;
-  const int wide = (tiles + 1) / 2;
+  // every row tile in one workgroup up to DENSE_MT of them, two even groups above; also where one
+  // group would leave half the CUs without a workgroup: 4096 x 4096 at 108 rows, one group -> two,
+  // fp16 24.1 -> 17.7 us, bf16 35.7 -> 24.1; 6144 x 4096 fp16 at 48 rows 18.6 -> 22.1
+  const int groups = row_tiles > DENSE_MT || (wide <= 128 && row_tiles > 2) ? 2 : 1;
   const dim3 grid((unsigned)(groups == 2 ? 16 * ((wide + 7) / 8) : wide));
   auto go = [&](auto mt) {
     hipLaunchKernelGGL((dense_gemv_wide<WT, 2, NW, decltype(mt)::value>), grid, dim3(NW * 64), 0, s,

@@ -11,9 +11,12 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("wt", [1, 2])
 # two row groups with a short second one and a partial last tile; column tiles past the last of
-# a workgroup; superblocks that do not divide over the waves (eight waves, then four)
+# a workgroup; superblocks that do not divide over the waves (eight waves, then four); the two
+# sides of the narrow outputs' rule (4096 columns) at two, three and five row tiles
 @pytest.mark.parametrize("M,N,K", [(17, 2064, 3072), (113, 2000, 2304), (129, 2032, 4096),
-                                   (145, 4112, 768), (250, 2050, 1024)])
+                                   (145, 4112, 768), (250, 2050, 1024), (32, 4096, 2304),
+                                   (17, 4112, 768), (33, 4096, 2048), (33, 4112, 2304),
+                                   (72, 4080, 768), (65, 4100, 4096)])
 def test_dense_gemv_wide_edges(gpu, wt, M, N, K):
     from snowllm_amd import layers as L, ops
     print(f"dense_gemv wide wt={wt} M={M} N={N} K={K}", flush=True)
