@@ -239,7 +239,10 @@ __global__ void __launch_bounds__(NW * 64) dense_gemv(const u32x4* __restrict__ 
     floatx4 scale = {1.f, 1.f, 1.f, 1.f};
     if constexpr (WT == WT_F16)
       scale = __builtin_bit_cast(floatx4, bload4(sr, vs, (uint32_t)(s * 16 * 4)));
-    __builtin_amdgcn_sched_barrier(0);  // every load of the superblock before its first product
+    // every load of the superblock before its first product: fp16, 9 rows, without -> with,
+    // 4096 x 4096 17.5 -> 10.9 us, 151,936 x 4096 225 -> 216, x 2048 (one superblock per wave)
+    // 113.8 -> 111.2; the last took 109.6 with the row tiles looped over in one workgroup
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int t = 0; t < NTILE; ++t) {
       floatx4 sb = {0.f, 0.f, 0.f, 0.f};
@@ -279,15 +282,15 @@ __global__ void __launch_bounds__(NW * 64) dense_gemv(const u32x4* __restrict__ 
 // wave's last superblock go out at out-of-range offsets and touch no memory. Bound: the weights'
 // bytes from HBM (nt loads, so that they do not displace the activations from L2) at two row
 // tiles; from there on L2, which every workgroup reads the activations from once per 32 columns:
-// 108 rows of a 151,936 x 4096 bf16 head read 5.6 GB in 447 us, 12.6 TB/s, with the vector units
-// 9 % and the matrix units about 25 % busy.
+// 108 rows of a 151,936 x 4096 fp16 head read 5.6 GB in 447 us, 12.6 TB/s, with the vector units
+// 9 % and the matrix units 13 % busy.
 // Two row tiles need few enough registers for two workgroups a CU (one, before): 151,936 x 2048
-// fp16 at 24 rows 134 -> 113 us, 151,936 x 4096 bf16 268 -> 244; rings
-// twice as deep instead: 150 us.
+// fp16 at 24 rows 134 -> 113 us, 151,936 x 4096 bf16 268 -> 244; rings twice as deep instead took
+// 150 us.
 // MI355X, 151,936 x 4096 fp16, us (four row tiles per workgroup, weights loaded a superblock at
 // a time, before): 36 rows 331 -> 300, 108 rows 710 -> 449, 256 rows 1503 -> 978; x 2048 bf16,
 // 108 rows 533 -> 378.
-// Two row groups (more than 8 row tiles) take the same columns 8 apart in dispatch order, so that
+// Two row groups take the same columns 8 apart in dispatch order, so that
 // both land on one XCD and the second's weights come from its L2.
 template <int WT, int NT, int NW, int MT>
 __global__ void __launch_bounds__(NW * 64)
@@ -607,8 +610,9 @@ __global__ void __launch_bounds__(WS * PPB * 64)
 // workgroup PG groups of P pairs (a gate and an up tile each), a group two waves that split the
 // superblocks as gate_up_kernel's do, each with both row tiles' products of every weight it
 // decodes; the waves exchange halves of their sums, so that each finishes one row tile. The same
-// products and sums, so the same bits, as gate_up_kernel per row tile. Bound: the vector units'
-// decode and rescaling and the L2 reads of the operands, as kquant_gemv_mt's; two row tiles by
+// products and sums, so the same bits, as gate_up_kernel per row tile. Bound: the L2 reads of the
+// operands (635 MB in 74 us at 108 rows of the size below, in a step) and the vector units' decode
+// and rescaling (37 % busy there), as kquant_gemv_mt's; two row tiles by
 // four column tiles are what the registers of two waves per SIMD hold (but for eleven of Q4_K, which
 // spill). F 14,336, K 4096, Q4_K, 108 rows: 66 us against 110 for seven 16-row launches.
 constexpr int GUR_PG = 4;
