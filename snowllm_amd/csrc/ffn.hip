@@ -612,7 +612,7 @@ __global__ void __launch_bounds__(WS * PPB * 64)
 // decodes; the waves exchange halves of their sums, so that each finishes one row tile. The same
 // products and sums, so the same bits, as gate_up_kernel per row tile. Bound: the L2 reads of the
 // operands (635 MB in 74 us at 108 rows of the size below, in a step) and the vector units' decode
-// and rescaling (37 % busy there), as kquant_gemv_mt's; two row tiles by
+// and rescaling (41 % busy there), as kquant_gemv_mt's; two row tiles by
 // four column tiles are what the registers of two waves per SIMD hold (but for eleven of Q4_K, which
 // spill). F 14,336, K 4096, Q4_K, 108 rows: 66 us against 110 for seven 16-row launches.
 constexpr int GUR_PG = 4;

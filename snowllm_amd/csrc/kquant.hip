@@ -93,8 +93,8 @@ __global__ void __launch_bounds__(NW * 64) kquant_gemv(const u32x4* __restrict__
 // operands of MT row tiles (gemv_rows_loop). Bound: the L2 reads (26 KB per 2 x 4 tiles and
 // superblock, 13 KB per 1 x 2) and the vector units' decode and rescaling, both shared by more
 // tiles the more a wave holds: Q4_K 2 x 4, 4096 x 14336, 126 rows, reads 388 MB from L2 in 33 us
-// (11.8 TB/s) with the vector units 48 % busy, Q6_K 1 x 2, 151,936 x 2048, 45 rows, 1.72 GB in
-// 150 us (11.4 TB/s) and 72 %. Two row tiles take the registers of two waves per SIMD, one
+// (11.8 TB/s) with the vector units 48 % busy; Q6_K 1 x 2, 151,936 x 2048, 45 rows, 1.72 GB in
+// 150 us (11.4 TB/s) and 72 %, its weights fetched into L2 once per row tile (767 MB). Two row tiles take the registers of two waves per SIMD, one
 // workgroup to a CU; one row tile is held to four waves per SIMD, two workgroups (above 128
 // registers Q8_0 took 10 to 15 % longer, 17.8 us against 15.3 at 5120 x 2048 and 128 rows). Q4_K
 // 4096 x 14336, 126 rows, with the operands' launch: 47 -> 38 us from HBM, 42 -> 32 repeated,
