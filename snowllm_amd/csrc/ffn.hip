@@ -240,8 +240,7 @@ __global__ void __launch_bounds__(NW * 64) dense_gemv(const u32x4* __restrict__ 
     if constexpr (WT == WT_F16)
       scale = __builtin_bit_cast(floatx4, bload4(sr, vs, (uint32_t)(s * 16 * 4)));
     // every load of the superblock before its first product: fp16, 9 rows, without -> with,
-    // 4096 x 4096 17.5 -> 10.9 us, 151,936 x 4096 225 -> 216, x 2048 (one superblock per wave)
-    // 113.8 -> 111.2; the last took 109.6 with the row tiles looped over in one workgroup
+    // 4096 x 4096 17.5 -> 10.9 us, 14,336 x 4096 27.4 -> 25.4
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int t = 0; t < NTILE; ++t) {
@@ -286,7 +285,8 @@ __global__ void __launch_bounds__(NW * 64) dense_gemv(const u32x4* __restrict__ 
 // 9 % and the matrix units 13 % busy.
 // Two row tiles need few enough registers for two workgroups a CU (one, before): 151,936 x 2048
 // fp16 at 24 rows 134 -> 113 us, 151,936 x 4096 bf16 268 -> 244; rings twice as deep instead took
-// 150 us.
+// 150 us. One row tile runs three: x 2048 fp16 at 9 rows 96 us, with two (and rings twice as deep)
+// 104, with four 111.
 // MI355X, 151,936 x 4096 fp16, us (four row tiles per workgroup, weights loaded a superblock at
 // a time, before): 36 rows 331 -> 300, 108 rows 710 -> 449, 256 rows 1503 -> 978; x 2048 bf16,
 // 108 rows 533 -> 378.
@@ -294,7 +294,7 @@ __global__ void __launch_bounds__(NW * 64) dense_gemv(const u32x4* __restrict__ 
 // both land on one XCD and the second's weights come from its L2.
 template <int WT, int NT, int NW, int MT>
 __global__ void __launch_bounds__(NW * 64)
-    __attribute__((amdgpu_waves_per_eu(MT == 2 ? 4 : 2, MT == 2 ? 4 : 2)))
+    __attribute__((amdgpu_waves_per_eu(MT == 1 ? 6 : MT == 2 ? 4 : 2, MT == 1 ? 6 : MT == 2 ? 4 : 2)))
 dense_gemv_wide(const u32x4* __restrict__ w, const void* __restrict__ act, void* __restrict__ c,
                 int M, int N, int S, int c_bf16, size_t tile_bytes, int groups) {
   constexpr int DX = 2, DW = MT == 8 && WT == WT_F16 ? 2 : 4;  // (there two spill six registers already)
@@ -1587,9 +1587,12 @@ int launch_dense(const void* w, const void* act, void* c, int M, int N, int S, i
   const size_t tb = xprep_tile_bytes(S);
   const int blocks = (tiles + NTILE - 1) / NTILE;
   const int wide = (tiles + 1) / 2;
-  if (row_tiles == 1 || blocks < 64 || (WT == WT_BF16 && row_tiles == 2 && wide <= 128)) {
+  if ((row_tiles == 1 && wide < 2048) || blocks < 64 || (WT == WT_BF16 && row_tiles == 2 && wide <= 128)) {
     // one row tile per workgroup: a narrow output (the router's 17 tiles) then still has
-    // workgroups for several CUs (the same sums per row tile). bf16 weights of up to 4096 columns
+    // workgroups for several CUs (the same sums per row tile). Up to 16 rows that is the faster
+    // form below 65,536 columns (bf16, 1 row, 14,336 x 4096 23.4 us against 24.5 in the wide form,
+    // 32,000 x 4096 45.0 and 46.8); a head's columns keep every CU busy with small waves and rings
+    // (151,936 x 2048, 1 row, fp16 102.1 us against 90.6, bf16 107.0 and 92.3). bf16 weights of up to 4096 columns
     // at two row tiles likewise: 4096 x 4096 at 24 rows 13.6 us, 14.6 in one workgroup of both;
     // 6144 x 4096 21.2 and 17.0
     hipLaunchKernelGGL((dense_gemv<WT, NTILE, NW>), dim3(blocks, row_tiles), dim3(NW * 64), 0, s,
@@ -1607,6 +1610,7 @@ int launch_dense(const void* w, const void* act, void* c, int M, int N, int S, i
                        (const u32x4*)w, act, c, M, N, S, c_bf16, tb, groups);
   };
   switch ((row_tiles + groups - 1) / groups) {
+    case 1: go(std::integral_constant<int, 1>{}); break;
     case 2: go(std::integral_constant<int, 2>{}); break;
     case 3: go(std::integral_constant<int, 3>{}); break;
     case 4: go(std::integral_constant<int, 4>{}); break;

@@ -44,6 +44,34 @@ def test_dense_gemv_wide_edges(gpu, wt, M, N, K):
     assert rel(out.cpu(), x.double().cpu() @ w.double().cpu().T) < K * 2.0 ** -24
 
 
+@pytest.mark.parametrize("wt", [1, 2])
+# up to 16 rows of a head's columns, at the edge of that rule: the bits of the narrow launches;
+# a lone last tile, a partial one, waves without a superblock, several superblocks per wave
+@pytest.mark.parametrize("M,N,K", [(1, 65520, 256), (9, 65521, 768), (16, 65536, 2304),
+                                   (13, 65550, 2048)])
+def test_dense_gemv_of_a_head(gpu, wt, M, N, K):
+    from snowllm_amd import layers as L, ops
+    print(f"dense_gemv head wt={wt} M={M} N={N} K={K}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    w = (torch.randn(N, K, device="cuda", generator=g) * 0.02).to(
+        torch.float16 if wt == 1 else torch.bfloat16)
+    x = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    x[0] *= 1e4   # rows of different operand scales
+    act = x
+    if wt == 1:
+        act = torch.empty(ops.gemm_kquant_a_ws_bytes(M, K), dtype=torch.uint8, device="cuda")
+        ops.gemm_kquant_prepare_a(x, act)
+    out = torch.full((M, N), float("nan"), device="cuda")
+    L.dense_gemv(wt, L.dense_shuffle(w), act, out, M, N, K)
+    for n0 in range(0, N, 32768):
+        n = min(32768, N - n0)
+        part = torch.empty(M, n, device="cuda")
+        L.dense_gemv(wt, L.dense_shuffle(w[n0:n0 + n].contiguous()), act, part, M, n, K)
+        assert torch.equal(out[:, n0:n0 + n], part)
+    # exact products summed in 32 bits: K roundings of 2^-24 at most
+    assert rel(out.cpu(), x.double().cpu() @ w.double().cpu().T) < K * 2.0 ** -24
+
+
 @pytest.mark.parametrize("m", [16, 33])
 def test_q6k_every_scale_is_exact(gpu, m):
     """Q6_K scales over the whole of int8 against quants 0, 63 and random ones: rows with a single
