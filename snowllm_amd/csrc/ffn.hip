@@ -279,8 +279,8 @@ __global__ void __launch_bounds__(NW * 64) dense_gemv(const u32x4* __restrict__ 
 // stream one 32-wide k-step at a time, the activations DX and the weights DW steps ahead (rings
 // in registers); the rows' scales wait in LDS for the end of their superblock. Loads past a
 // wave's last superblock go out at out-of-range offsets and touch no memory. Bound: the weights'
-// bytes from HBM (nt loads, so that they do not displace the activations from L2) at two row
-// tiles; from there on L2, which every workgroup reads the activations from once per 32 columns:
+// bytes from HBM (nt loads, so that they do not displace the activations from L2) up to two row
+// tiles (151,936 x 2048 fp16, 9 rows: 6.8 TB/s); from there on L2, which every workgroup reads the activations from once per 32 columns:
 // 108 rows of a 151,936 x 4096 fp16 head read 5.6 GB in 447 us, 12.6 TB/s, with the vector units
 // 9 % and the matrix units 13 % busy.
 // Two row tiles need few enough registers for two workgroups a CU (one, before): 151,936 x 2048
